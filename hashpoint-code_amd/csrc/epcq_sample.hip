@@ -20,9 +20,14 @@
 #include <mutex>
 
 #include "epcq_common.h"
+#include "epcq_rows.h"
 #include "epcq_sampler.h"
 
 namespace epcq {
+// Defined in epcq_rows_kernels.h, instantiated in epcq_rows_inst_*.hip.
+template <int MODE, int KMAX>
+void launch_rows(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
+                 hipStream_t st);
 // Defined in epcq_sample_kernels.h, instantiated in epcq_sample_inst_*.hip
 // (NW = 1) and epcq_sample_wide_*.hip (NW = 4).
 template <int MODE, int KMAX, int SMAX, int NW>
@@ -94,18 +99,27 @@ epcq_tuning current_tuning() {
 // Pixel-ordered copy of the points, one thread per list position: (x, y,
 // z, index bits) and, with per-point radii, the radius's squared threshold.
 // Positions holding no valid index (the -1 tail) are left alone; the hash
-// entries never point there.
+// entries never point there.  cand: the points' candidate bounds for the
+// row-run sampler (uniform radius r0 without prad); queue: the deferred-ray queue that the row-run
+// that sampler starts from, emptied here.
 __global__ __launch_bounds__(kBlock) void point_copy_kernel(const int* __restrict__ sorted_idx,
                                                             const float* __restrict__ xyz,
                                                             const float* __restrict__ radius, int64_t n,
-                                                            float4* __restrict__ pts, float* __restrict__ prad) {
+                                                            float4* __restrict__ pts, float* __restrict__ prad,
+                                                            float4* __restrict__ cand, float r0,
+                                                            const float* __restrict__ c2w,
+                                                            RowQueue* __restrict__ queue) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0 && queue) queue->count = 0;
     if (i >= n) return;
     const int id = sorted_idx[i];
     if (id < 0 || id >= n) return;
     const float* q = xyz + 3 * (int64_t)id;
-    pts[i] = make_float4(q[0], q[1], q[2], __int_as_float(id));
-    if (prad) prad[i] = point_threshold(radius[id]);
+    const float4 p = make_float4(q[0], q[1], q[2], __int_as_float(id));
+    pts[i] = p;
+    float lim = 0.0f;
+    if (prad) prad[i] = lim = point_threshold(radius[id]);
+    if (cand) cand[i] = row_candidate(row_frame(c2w), p, prad ? __builtin_amdgcn_sqrtf(lim) : r0);
 }
 
 // Bucket cones, one thread per pixel: from the pixel-ordered copy pts_in
@@ -241,14 +255,84 @@ SampleOpts make_opts(const float* xyz, const epcq_options* opt, const float* rad
     return o;
 }
 
+size_t sampling_bytes(int64_t n, int64_t P);
+
+// Whether a ray list takes the one-wave-per-ray form over row runs
+// (epcq_rows_wave.h): under the same bounds, lists of at most list_wave rays.
+int takes_rows_list(const SampleOpts& o, int64_t R, int live_bound) {
+    return o.k <= kRowMaxK && live_bound <= 2 && R <= o.list_wave ? kRowsWave : kRowsNone;
+}
+
+// Which form an image takes, by its pixels P and the points d that a ray's
+// window holds on average (measured with the build; tile form / wave form /
+// lane sets in ms):
+// - P <= kWaveImage: 64 rays per wave would leave SIMDs idle; waves.  1M points
+//   at 400 x 300, k = 5: 0.60 / 0.35 / 1.18; at 640 x 512: 0.47 / 0.69 / 1.1.
+// - up to four times as many: each tile is a long serial walk, and the longest
+//   ones end last.  Waves from kWaveDense points on (half the pixels: from
+//   kWaveMid): a sphere at 500 x 503, k = 7: d = 195 1.15 / 0.71 / 1.03, d =
+//   292 1.53 / 0.81 / 1.47; a box at 640 x 480, k = 7: d = 160 0.64 / 0.97 /
+//   0.92, d = 319 1.15 / 1.26 / 1.62; d = 4400 10.6 / 6.2 / 8.0.
+// - windows of more than eight columns, two blocks of whose tiles fit on a CU,
+//   cost more in both forms, and up to four times as many pixels (from 13
+//   columns on eight times) the lane sets are ahead from kWaveMid to kWaveWide
+//   points: k = 9 at 500 x 503, d = 298
+//   0.86 / 1.04 / 0.89 in a box and 1.92 / 0.88 / 1.02 on a sphere; k = 11 at
+//   640 x 480, d = 364 1.34 / 1.40 / 1.19; k = 15 at 800 x 800, d = 351 1.67 /
+//   - / 1.52; but k = 9 at 800 x 800, d = 253 2.27 / - / 2.82, at 500 x 503, d =
+//   484 3.59 / 1.01 / 1.53, and k = 15 at 1920 x 1080, d = 217 2.66 / - / 5.56.
+constexpr int64_t kWaveImage = 131072;
+constexpr int64_t kWaveMid = 100;
+constexpr int64_t kWaveDense = 256;
+constexpr int64_t kWaveWide = 400;
+
+// Where a window holds fewer than ten points on average, a ray has next to
+// nothing to test, and the rows' bounds and the S * K slots of the dense
+// layout are what is left: there the lane sets stay ahead.  Measured, rows
+// against lane sets, 800 x 800 pixels, k = 5, dense layout: 0.19 against 0.16
+// ms with 100k points, 0.24 against 0.21 with 200k, 0.27 against 0.26 with
+// 300k, 0.33 against 0.39 with 600k; in the compact layout rows are ahead at
+// each of these (200k points at 1600 x 1200, k = 3: 0.31 against 0.36).
+constexpr int64_t kRowsSparse = 10;
+
+// Whether a full image takes the row-run sampler (epcq_rows.h): windows that
+// its LDS rows hold, options under which a ray can visit two slots at most
+// (with per-point radii the caller's s_max stands for that bound; a ray that
+// visits more is run by a whole wave), and a workspace for the point copy and
+// the queue of deferred rays.
+int takes_rows(SampleOpts& o, const epcq_camera* cam, int64_t n, int live_bound, bool compact,
+               const void* workspace, size_t workspace_bytes) {
+    const int64_t P = (int64_t)cam->width * cam->height;
+    if (o.k > kRowMaxK || live_bound > 2 || !workspace || workspace_bytes < sampling_bytes(n, P)) return kRowsNone;
+    const int64_t d = (int64_t)o.L * n / std::max<int64_t>(P, 1);
+    // candidates that the launch gives a lane of each SIMD: a ray with far more
+    // would outlast the others
+    o.row_heavy = (int)std::min<int64_t>(kRowHeavyMost, std::max<int64_t>(kRowHeavyLeast, (int64_t)o.L * n / (65536 * 128)));
+    if (P <= kWaveImage) return kRowsWave;
+    if (!compact && d < kRowsSparse) return kRowsNone;
+    if (o.k > 8) {
+        if (P <= 4 * kWaveImage && d >= kWaveWide) return kRowsWave;
+        if (P <= (o.k > 12 ? 8 : 4) * kWaveImage && d >= kWaveMid && d < kWaveWide) return kRowsNone;
+        return kRowsTiles;
+    }
+    if (P <= 4 * kWaveImage && d >= (P <= 2 * kWaveImage ? kWaveMid : kWaveDense)) return kRowsWave;
+    return kRowsTiles;
+}
+
 ViewArgs make_view(const epcq_camera* cam, const int* sorted_idx, const int* hash) {
     return ViewArgs{cam->c2w, cam->fx, cam->fy, cam->cx, cam->cy, cam->width, cam->height,
-                    reinterpret_cast<const int2*>(hash), sorted_idx, nullptr, nullptr, nullptr, nullptr, nullptr};
+                    reinterpret_cast<const int2*>(hash), sorted_idx, nullptr, nullptr, nullptr, nullptr, nullptr,
+                    nullptr};
 }
 
 // Workspace layout of the samplers: cone_a [P] float4 | cone_b [P] float2 |
-// pixel-ordered points [n] float4 | pixel-ordered radii [n] float.
+// pixel-ordered points [n] float4 | pixel-ordered radii [n] float | candidate
+// bounds [n + kRowPad] float4.
 size_t cone_bytes(int64_t P) { return align_up((size_t)P * 16, 256) + align_up((size_t)P * 8, 256); }
+
+size_t sampling_bytes(int64_t n, int64_t P) {
+    return cone_bytes(P) + align_up((size_t)n * 16, 256) + align_up((size_t)n * 4, 256) + (size_t)(n + kRowPad) * 16;
+}
 
 // Bucket cones and the pixel-ordered point copy in the workspace (when it is
 // large enough: then o.cull is set and view reads them).  They cost a pass
@@ -266,6 +350,26 @@ void prepare_bounds(SampleOpts& o, ViewArgs& view, int64_t n, const epcq_camera*
     o.cull = 0;
     if (!workspace || workspace_bytes < cone_bytes(P)) return;
     if (rays >= 0 && rays * o.L * kConeVisitRatio < P) return;
+    if (o.rows) {
+        // the row-run sampler: point copy and candidate bounds, and the queue
+        // in the cones' place (a ray list makes do with the copy alone)
+        const size_t pts_off = cone_bytes(P), rad_off = pts_off + align_up((size_t)n * 16, 256);
+        const size_t cand_off = rad_off + align_up((size_t)n * 4, 256);
+        if (workspace_bytes < rad_off) return;
+        char* w = static_cast<char*>(workspace);
+        float4* pts = reinterpret_cast<float4*>(w + pts_off);
+        float* prad = o.radius && workspace_bytes >= rad_off + (size_t)n * 4 ? reinterpret_cast<float*>(w + rad_off)
+                                                                            : nullptr;
+        float4* cand = workspace_bytes >= sampling_bytes(n, P) ? reinterpret_cast<float4*>(w + cand_off) : nullptr;
+        RowQueue* queue = reinterpret_cast<RowQueue*>(w);
+        point_copy_kernel<<<dim3((unsigned)ceil_div(std::max<int64_t>(n, 1), kBlock)), dim3(kBlock), 0, st>>>(
+            sorted_idx, o.xyz, o.radius, n, pts, prad, cand, std::sqrt(o.r2lim), cam->c2w, queue);
+        view.cone_a = reinterpret_cast<const float4*>(queue);
+        view.pts = pts;
+        view.prad = prad;
+        view.cand = cand;
+        return;
+    }
     char* w = static_cast<char*>(workspace);
     float4* ca = reinterpret_cast<float4*>(w);
     float2* cb = reinterpret_cast<float2*>(w + align_up((size_t)P * 16, 256));
@@ -277,7 +381,8 @@ void prepare_bounds(SampleOpts& o, ViewArgs& view, int64_t n, const epcq_camera*
         // the copy first, in parallel over list positions, then the cones from it
         if (n > 0)
             point_copy_kernel<<<dim3((unsigned)ceil_div(n, kBlock)), dim3(kBlock), 0, st>>>(sorted_idx, o.xyz,
-                                                                                          o.radius, n, pts, prad);
+                                                                                          o.radius, n, pts, prad,
+                                                                                          nullptr, 0.0f, nullptr, nullptr);
         bucket_cone_kernel<<<dim3((unsigned)ceil_div(P, kBlock)), dim3(kBlock), 0, st>>>(
             reinterpret_cast<const int2*>(hash), nullptr, nullptr, pts, o.radius, o.r0, cam->c2w, P, ca, cb, nullptr,
             nullptr);
@@ -308,12 +413,36 @@ void launch_smax(const SampleOpts& o, const SampleOut& out, const ViewArgs& view
     }
 }
 
+// Feature sums of the compact rows after the row-run sampler.
+void launch_idw_rows(const SampleOpts& o, const SampleOut& out, int64_t R, hipStream_t st) {
+    const int64_t rows = R * out.s_max;
+    int G = 1;  // lanes per row: a power of two, at most 32, about one per four features
+    while (G < 32 && 4 * G < o.F) G *= 2;
+    const dim3 grid((unsigned)ceil_div(rows, 256 / G)), block(256);
+    if (o.feat_bf16 && o.feat_vec)
+        idw_rows_kernel<true, true><<<grid, block, 0, st>>>(o.feat, o.F, G, rows, o.Kc, out.nb_idx, out.w, out.agg);
+    else if (o.feat_bf16)
+        idw_rows_kernel<true, false><<<grid, block, 0, st>>>(o.feat, o.F, G, rows, o.Kc, out.nb_idx, out.w, out.agg);
+    else if (o.feat_vec)
+        idw_rows_kernel<false, true><<<grid, block, 0, st>>>(o.feat, o.F, G, rows, o.Kc, out.nb_idx, out.w, out.agg);
+    else
+        idw_rows_kernel<false, false><<<grid, block, 0, st>>>(o.feat, o.F, G, rows, o.Kc, out.nb_idx, out.w, out.agg);
+}
+
 // `bound`: samples of one ray that are stored (kernels with a bound of 2 keep
 // two sample depths in registers; the others keep kRegSamples and re-read
 // later ones from the outputs).
 int launch_sample(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
                   int mode, int bound, hipStream_t st, const char* who) {
     if (R == 0) return EPCQ_OK;
+    if (o.rows) {
+        if (mode == EPCQ_MODE_COMPAT) launch_rows<EPCQ_MODE_COMPAT, kCompatBuffer>(o, out, view, rays, R, st);
+        else if (o.Kc <= 8) launch_rows<EPCQ_MODE_KNN, 8>(o, out, view, rays, R, st);
+        else if (o.Kc <= 16) launch_rows<EPCQ_MODE_KNN, 16>(o, out, view, rays, R, st);
+        else launch_rows<EPCQ_MODE_KNN, 32>(o, out, view, rays, R, st);
+        if (o.feat && o.rows == kRowsTiles) launch_idw_rows(o, out, R, st);  // the wave form sums the features itself
+        return check_launch(who);
+    }
     const epcq_tuning tu = current_tuning();
     const TilePlan tp = plan_tiles(o.k, tu.tile_w, tu.tile_h, tu.tile_cap, tu.flags, o.radius != nullptr);
     if (mode == EPCQ_MODE_COMPAT) {
@@ -372,7 +501,7 @@ extern "C" int32_t epcq_max_live_samples(const epcq_options* opt, float r_max) {
 
 extern "C" size_t epcq_sampling_workspace_size(int64_t n, int32_t height, int32_t width) {
     if (height <= 0 || width <= 0 || n < 0) return 0;
-    return cone_bytes((int64_t)height * width) + align_up((size_t)n * 16, 256) + (size_t)n * 4;
+    return sampling_bytes(n, (int64_t)height * width);
 }
 
 extern "C" int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camera* cam, const epcq_options* opt,
@@ -389,6 +518,7 @@ extern "C" int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camer
     if (opt->num_sample_points_per_ray == 0) return EPCQ_OK;
     const int bound = epcq_max_live_samples(opt, opt->radius_threshold);
     SampleOpts o = make_opts(xyz, opt, nullptr);
+    o.rows = takes_rows(o, cam, n, bound, false, workspace, workspace_bytes);
     SampleOut out{};
     out.sp_xyz = sp_xyz;
     out.pc_idx = pc_idx;
@@ -417,6 +547,7 @@ extern "C" int epcq_quick_sampling_rays(const float* xyz, int64_t n, const epcq_
     if (opt->num_sample_points_per_ray == 0 || R == 0) return EPCQ_OK;
     const int bound = epcq_max_live_samples(opt, opt->radius_threshold);
     SampleOpts o = make_opts(xyz, opt, nullptr);
+    o.rows = takes_rows_list(o, R, bound);
     SampleOut out{};
     out.sp_xyz = sp_xyz;
     out.pc_idx = pc_idx;
@@ -460,6 +591,8 @@ extern "C" int epcq_knn_sampling(const float* xyz, int64_t n, const epcq_camera*
     out.w = w;
     out.agg = agg;
     const int64_t nr = rays ? R : (int64_t)cam->width * cam->height;
+    const int live = radius ? s_max : epcq_max_live_samples(opt, opt->radius_threshold);
+    o.rows = rays ? takes_rows_list(o, nr, live) : takes_rows(o, cam, n, live, true, workspace, workspace_bytes);
     hipStream_t st = as_stream(stream);
     ViewArgs view = make_view(cam, sorted_idx, hash);
     prepare_bounds(o, view, n, cam, sorted_idx, hash, workspace, workspace_bytes, rays ? R : -1, st);

@@ -72,6 +72,8 @@ struct SampleOpts {
     int cull;             // skip neighbour buckets by their bounding spheres
     int heavy;            // a ray whose hit lanes hold more candidates is run by its whole wave (0: never)
     int list_wave;        // ray lists of at most this many rays run one wave per ray (0: never)
+    int row_heavy;        // the row-run tiles' factor on heavy
+    int rows;             // row-run sampler (epcq_rows.h): kRowsNone, kRowsTiles or kRowsWave
 };
 
 struct SampleOut {
@@ -1463,6 +1465,7 @@ struct ViewArgs {
     const float4* pts;     // pixel-ordered points (bucket_cone_body) or nullptr
     const float* prad;     // pixel-ordered radius thresholds (per-point radius) or nullptr
     const float* xyz;      // the view's cloud (nullptr: SampleOpts::xyz)
+    const float4* cand;    // pixel-ordered candidate bounds (row_candidate) or nullptr
 };
 
 __device__ __forceinline__ void view_ray(const ViewArgs& v, int u, int vv, Ray& ray) {
