@@ -24,10 +24,6 @@
 #include "epcq_sampler.h"
 
 namespace epcq {
-// Defined in epcq_rows_kernels.h, instantiated in epcq_rows_inst_*.hip.
-template <int MODE, int KMAX>
-void launch_rows(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
-                 hipStream_t st);
 // Defined in epcq_sample_kernels.h, instantiated in epcq_sample_inst_*.hip
 // (NW = 1) and epcq_sample_wide_*.hip (NW = 4).
 template <int MODE, int KMAX, int SMAX, int NW>
@@ -399,12 +395,13 @@ void prepare_bounds(SampleOpts& o, ViewArgs& view, int64_t n, const epcq_camera*
 }
 
 // Windows of more than 64 lanes (k > 8) take the kernels with 4-word lane
-// sets (exact culling up to k = 16; larger windows visit every lane).
+// sets (exact culling up to k = 16; larger windows visit every lane).  The
+// row-run sampler has one form for all of them.
 template <int MODE, int KMAX>
 void launch_smax(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
                  const TilePlan& tp, int bound, hipStream_t st) {
-    const bool wide = o.L > 64;
-    if (bound <= 2) {
+    const bool wide = o.L > 64 && !o.rows;
+    if (bound <= 2 || o.rows) {
         if (wide) launch_lay<MODE, KMAX, 2, 4>(o, out, view, rays, R, tp, st);
         else launch_lay<MODE, KMAX, 2, 1>(o, out, view, rays, R, tp, st);
     } else {
@@ -435,14 +432,6 @@ void launch_idw_rows(const SampleOpts& o, const SampleOut& out, int64_t R, hipSt
 int launch_sample(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
                   int mode, int bound, hipStream_t st, const char* who) {
     if (R == 0) return EPCQ_OK;
-    if (o.rows) {
-        if (mode == EPCQ_MODE_COMPAT) launch_rows<EPCQ_MODE_COMPAT, kCompatBuffer>(o, out, view, rays, R, st);
-        else if (o.Kc <= 8) launch_rows<EPCQ_MODE_KNN, 8>(o, out, view, rays, R, st);
-        else if (o.Kc <= 16) launch_rows<EPCQ_MODE_KNN, 16>(o, out, view, rays, R, st);
-        else launch_rows<EPCQ_MODE_KNN, 32>(o, out, view, rays, R, st);
-        if (o.feat && o.rows == kRowsTiles) launch_idw_rows(o, out, R, st);  // the wave form sums the features itself
-        return check_launch(who);
-    }
     const epcq_tuning tu = current_tuning();
     const TilePlan tp = plan_tiles(o.k, tu.tile_w, tu.tile_h, tu.tile_cap, tu.flags, o.radius != nullptr);
     if (mode == EPCQ_MODE_COMPAT) {
@@ -454,6 +443,7 @@ int launch_sample(const SampleOpts& o, const SampleOut& out, const ViewArgs& vie
     } else {
         launch_smax<EPCQ_MODE_KNN, 32>(o, out, view, rays, R, tp, bound, st);
     }
+    if (o.feat && o.rows == kRowsTiles) launch_idw_rows(o, out, R, st);  // the wave form sums the features itself
     return check_launch(who);
 }
 

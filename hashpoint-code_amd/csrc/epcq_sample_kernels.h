@@ -120,14 +120,24 @@ void launch_one(const SampleOpts& o, const SampleOut& out, const ViewArgs& view,
     launch_kernels<MODE, KMAX, SMAX, LAY, false, NW>(o, out, view, rays, R, tp, st);
 }
 
+// Row-run kernels (epcq_rows_kernels.h), instantiated in epcq_rows_inst_*.hip.
+template <int MODE, int KMAX>
+void launch_rows(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
+                 hipStream_t st);
+
 template <int MODE, int KMAX, int SMAX, int NW>
 void launch_lay(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
                 const TilePlan& tp, hipStream_t st) {
+    if constexpr (SMAX == 2 && NW == 1) {
+        if (o.rows) {
+            launch_rows<MODE, KMAX>(o, out, view, rays, R, st);
+            return;
+        }
+    }
     if (out.sp_xyz) launch_one<MODE, KMAX, SMAX, kLayDense, NW>(o, out, view, rays, R, tp, st);
     else if (o.feat) launch_one<MODE, KMAX, SMAX, kLayFeat, NW>(o, out, view, rays, R, tp, st);
     else launch_one<MODE, KMAX, SMAX, kLayCompact, NW>(o, out, view, rays, R, tp, st);
 }
-
 
 }  // namespace epcq
 
