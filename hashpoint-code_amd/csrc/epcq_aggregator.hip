@@ -18,19 +18,30 @@
 //   xc    = [sum_k w_k h4_k, PE(d, 4)]                        280
 //   rgb   = sigmoid(C4 lrelu(C3 lrelu(C2 lrelu(C1 xc + c1) + c2) + c3) + c4) * 1.002 - 0.001
 //
-// Layout.  Pairs are rows r = m * Kp + k of a virtual [M, Kp] grid, Kp the
-// power of two >= K (rows with k >= K are invalid), so that 32 consecutive
-// rows -- one wave's strip -- hold whole samples.  A wave runs its strip
-// through all four point layers with the activations in its own LDS region
-// (32 rows of bf16), each layer a 32 x N tile sequence of
-// v_mfma_f32_32x32x16_bf16 whose B operand (the weight rows, [N, K] bf16
-// row-major, zero-padded to a multiple of 16 inputs) streams from L2; the
-// epilogue adds the bias, applies the activation and writes bf16 back over
-// the layer's input rows.  The strip then reduces its samples in LDS and
-// writes each sample's colour-branch input (bf16, 288 wide) to the
-// workspace; a second kernel runs the colour MLP over strips of 32 samples.
-// Nothing is accumulated across waves, so results do not depend on
-// scheduling.
+// Layout.  Each layer is computed transposed, Y^T = W X^T, with the weights as
+// the left operand of v_mfma_f32_32x32x16_bf16: a lane then owns one row of the
+// batch in every layer (its column of the result), and the accumulators of one
+// layer become the right operands of the next by a conversion to bf16 and a
+// swap of lane halves (v_permlane32_swap), so activations never leave the
+// registers.  A block is four waves of 32 rows; the weights stream from L2
+// through LDS in pieces of 64 outputs, copied by the load unit itself
+// (global_load_lds) into one buffer while the waves multiply from the other,
+// with one barrier per piece.  Two blocks fit on a CU and drift apart, so one's
+// encodings, epilogues and reductions run under the other's matrix products.
+//
+// Pairs are rows: a block takes 128 / K whole samples, rows in order, whichever
+// wave they fall to (K = 5 fills 125 of 128 rows).  At the end the rows' last
+// activations go to LDS and each half of a wave reduces one sample after
+// another into the workspace (bf16, 256 wide); a second kernel runs the colour
+// MLP, a row per sample.  Nothing is accumulated across waves, so results do
+// not depend on scheduling.
+//
+// What bounds it: the matrix cores, at the clock that they leave (about 1.7 of
+// 2.4 GHz), for two thirds of a block's time, then the encodings and
+// reductions.  Measured, both kernels, against weight chunks of 16 inputs that
+// passed through registers, activations in LDS and rows padded to a power of
+// two: 1.28M samples of 8 neighbours 7.9 -> 5.9 ms, 100k of 9 1.19 -> 0.58,
+// 100k of 5 0.68 -> 0.37, 20k of 8 0.20 -> 0.14.
 #include <math.h>
 
 #include <type_traits>
@@ -44,14 +55,17 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWave = 64;
-constexpr int kStrip = 32;              // rows per wave
-constexpr int kWavesPerBlock = 4;          // colour kernel
-constexpr int kBlock = kWave * kWavesPerBlock;
-constexpr int kPairWaves = 8;              // pair kernel: 256 rows share each weight chunk
-constexpr int kPairBlock = kWave * kPairWaves;
-constexpr int kLdsStride = 296;         // bf16 per LDS row (288 + 8: rows start on different banks)
+constexpr int kWaves = 4;
+constexpr int kBlock = kWave * kWaves;
+constexpr int kWaveRows = 32;
+constexpr int kRows = kWaves * kWaveRows;  // rows of a block
 constexpr int kFeat = 32;               // F: block1 takes 7F + 60 = 284 inputs
 constexpr int kX1 = 288, kH = 256, kX3 = 272, kXc = 288, kC = 128;
+constexpr int kPieceTiles = 2;          // tiles of 32 outputs in a weight piece
+constexpr int kPiece = 32 * kPieceTiles;
+constexpr int kPieceBytes = kPiece * kX1 * 2;  // the longest rows
+constexpr int kLdsStride = kH + 8;      // bf16 per row of last activations (8: rows start on different banks)
+static_assert(2 * kWaveRows * kLdsStride * 2 <= kPieceBytes, "a buffer holds two waves' rows");
 
 // Round to nearest even (the hardware conversion, v_cvt_pk_bf16_f32).
 __device__ __forceinline__ uint16_t to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
@@ -93,14 +107,10 @@ __device__ __forceinline__ void pe_double(float s, float c, float& s2, float& c2
 __device__ __forceinline__ float from_bf16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // v for v > 0, else 0.01 v, as the larger of the two: one multiply and one
-// v_max_f32, written out because fmaxf of a matrix-core result adds a
-// NaN-quieting max of its own.  Equal to the compare-and-select form for every
-// finite v, +-0 and +-inf (a NaN stays a NaN).
-__device__ __forceinline__ float lrelu(float v) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(v), "v"(0.01f * v));
-    return r;
-}
+// v_maximum3_f32 (fmaxf of a matrix-core result adds a NaN-quieting max of its
+// own).  Equal to the compare-and-select form for every finite v, +-0 and
+// +-inf (a NaN stays a NaN).
+__device__ __forceinline__ float lrelu(float v) { return __builtin_elementwise_maximum(v, 0.01f * v); }
 
 // torch.nn.Softplus(beta=1, threshold=20)
 __device__ __forceinline__ float softplus(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
@@ -111,128 +121,182 @@ __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     return v;
 }
 
-// One layer over the wave's strip: out[32, 32 NT] = act(in[32, 16 KS] W^T + b)
-// with W [32 NT, 16 KS] bf16 row-major.  `io` is the strip's LDS rows; the
-// output overwrites columns [0, 32 NT) of the same rows once every input has
-// been read.  The 32x32x16 operands: lane l holds A[l % 32][8 (l / 32) + v]
-// and B[8 (l / 32) + v][l % 32], v < 8; accumulator register r of lane l is
-// D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
-template <int KS, int NT, bool LEAKY>
-__device__ __forceinline__ void strip_layer(uint16_t* io, const uint16_t* __restrict__ W,
-                                            const float* __restrict__ bias) {
-    const int lane = threadIdx.x % kWave;
-    const int row = lane & 31;
-    const int kh = (lane >> 5) * 8;
-    constexpr int K = 16 * KS;
-    // every accumulator of tile t in this lane is output column 32 t + row:
-    // it starts at that column's bias
-    f32x16 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = (f32x16)(bias[t * 32 + row]);
-    const uint16_t* a_row = io + row * kLdsStride + kh;
-    const uint16_t* w_row = W + (size_t)row * K + kh;
-    // the weight operands of steps ks + 1 and ks + 2 load while step ks
-    // multiplies (they come from L2: two steps cover its latency)
-    bf16x8 b0[NT], b1[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        b0[t] = load8(w_row + (size_t)t * 32 * K);
-        b1[t] = load8(w_row + (size_t)t * 32 * K + (KS > 1 ? 16 : 0));
+// The eights (a0, a1 | a2, a3) of which each lane half holds half (two packed
+// registers each): half 0 gets the whole first eight, half 1 the second.
+__device__ __forceinline__ bf16x8 swap_halves(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1) {
+    const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
+    const auto s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+    return __builtin_bit_cast(bf16x8, make_uint4(s0[0], s1[0], s0[1], s1[1]));
+}
+
+// Copies outputs [n0, n0 + 64) of the weights W [N, 16 KS] to `buf`; complete
+// after the next __syncthreads().  Each wave takes 16 rows, 64 bytes of them at
+// a time (two steps of 16 inputs; of an odd last one, what follows it in memory
+// or zeros, which nobody reads).  The load unit writes a lane's 16 bytes at
+// slot `lane` of the instruction's 1024; the lane picks its piece of the row by
+// a rotation (an exclusive or with half its row), so that the eight lanes of a
+// read cycle, eight rows at one input step, find theirs on different banks.
+// ALIGNED: W is 16-byte aligned; else the copies go through registers.
+template <int KS, int N, bool ALIGNED>
+struct Fetch {
+    static constexpr int kSteps = (KS + 1) / 2;
+    static constexpr int K = 16 * KS;
+    const uint16_t* W;
+    int at;      // the lane's first input
+    uint4* dst;  // the wave's part of the buffer
+
+    __device__ __forceinline__ Fetch(const uint16_t* w, int n0, uint4* buf) : W(w) {
+        const int lane = threadIdx.x % kWave;
+        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+        at = (n0 + wave * 16 + lane / 4) * K + ((lane ^ (lane / 8)) & 3) * 8;
+        dst = buf + wave * kSteps * kWave;
     }
-#pragma unroll 1
-    for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8 a = load8(a_row + ks * 16);
-        const int kn = (ks + 2 < KS ? ks + 2 : KS - 1) * 16;
-        bf16x8 bn[NT];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) bn[t] = load8(w_row + (size_t)t * 32 * K + kn);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0[t], acc[t], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            b0[t] = b1[t];
-            b1[t] = bn[t];
+    // the 64 bytes of steps 2 i and 2 i + 1
+    __device__ __forceinline__ void step(int i) const {
+        if (i >= kSteps) return;
+        if (ALIGNED) {
+            // a buffer load: one that goes through a flat address would make
+            // every LDS read wait for all others
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(W), 0, N * K * 2, 0x00020000);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + i * kWave), 16,
+                                                     2 * at, 64 * i, 0, 0);
+        } else {
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (at + 32 * i < N * K) __builtin_memcpy(&v, W + at + 32 * i, sizeof(v));
+            dst[i * kWave + threadIdx.x % kWave] = v;
         }
     }
-    const int r0 = (lane >> 5) * 4;
+    __device__ __forceinline__ void all() const {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int c = t * 32 + row;
+        for (int i = 0; i < kSteps; ++i) step(i);
+    }
+};
+
+struct NoFetch {
+    static constexpr int kSteps = 0;
+    __device__ __forceinline__ NoFetch(const uint16_t*, int, uint4*) {}
+    __device__ __forceinline__ void step(int) const {}
+};
+
+// The lane's weight operand of tile t at step ks.
+template <int KS>
+__device__ __forceinline__ bf16x8 weight_operand(const uint4* w, int t, int ks) {
+    const int lane = threadIdx.x % kWave;
+    const int row = lane & 31;
+    const int slot = (row & 15) * 4 + ((((ks & 1) << 1) + (lane >> 5)) ^ ((row >> 1) & 3));
+    return __builtin_bit_cast(bf16x8, w[(row >> 4) * ((KS + 1) / 2 * kWave) + slot + (2 * t * ((KS + 1) / 2) + ks / 2) * kWave]);
+}
+
+// The accumulators of a piece of 64 outputs.
+typedef f32x16 PieceAcc[kPieceTiles];
+
+// Activation and conversion of a quarter (16 outputs) of a finished piece: an
+// operand of the next layer.
+__device__ __forceinline__ bf16x8 finish_quarter(const PieceAcc& acc, int c) {
+    uint32_t p[4];
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            // rows rr and rr + 1 of column c: one conversion for both
-            const int rr = (r >> 2) * 8 + r0 + (r & 3);
-            float v0 = acc[t][r], v1 = acc[t][r + 1];
-            if (LEAKY) v0 = lrelu(v0), v1 = lrelu(v1);
-            const uint32_t p = pack_bf16(v0, v1);
-            io[rr * kLdsStride + c] = (uint16_t)p;
-            io[(rr + 1) * kLdsStride + c] = (uint16_t)(p >> 16);
+    for (int q = 0; q < 4; ++q)
+        p[q] = pack_bf16(lrelu(acc[c / 2][8 * (c % 2) + 2 * q]), lrelu(acc[c / 2][8 * (c % 2) + 2 * q + 1]));
+    return swap_halves(p[0], p[1], p[2], p[3]);
+}
+__device__ __forceinline__ void finish_piece(const PieceAcc& acc, bf16x8* y) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) y[c] = finish_quarter(acc, c);
+}
+
+// The biases of 64 outputs, where the accumulators start.
+__device__ __forceinline__ void start_piece(PieceAcc& acc, const float* s_bias) {
+    const int half = threadIdx.x % kWave >> 5;
+#pragma unroll
+    for (int t = 0; t < kPieceTiles; ++t) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 b = *reinterpret_cast<const float4*>(s_bias + 32 * t + 8 * q + 4 * half);
+            acc[t][4 * q] = b.x;
+            acc[t][4 * q + 1] = b.y;
+            acc[t][4 * q + 2] = b.z;
+            acc[t][4 * q + 3] = b.w;
         }
     }
 }
 
-// strip_layer for the pair kernel's 256-wide layers, with the weight rows
-// staged through LDS for the whole block: step ks of the K loop multiplies
-// the chunk W[:, 16 ks, 16 ks + 16) (8 KB), which the block's 512 threads
-// copy from L2 into s_w, 16 bytes each, two steps ahead through registers.
-// Every wave of the block calls it (it holds block barriers); `active`
-// waves multiply, the others only help with the copies.
-template <int KS>
-__device__ __forceinline__ void block_layer(uint16_t* io, uint16_t* s_w, const uint16_t* __restrict__ W,
-                                            const float* __restrict__ bias, bool active) {
-    constexpr int K = 16 * KS;
-    constexpr int NT = kH / 32;
-    static_assert(KS >= 2, "two chunks in flight");
-    static_assert(kPairBlock == 2 * kH, "one 16-byte piece of the chunk per thread");
-    const int tid = threadIdx.x;
-    const int lane = tid % kWave;
-    const int row = lane & 31;
-    const int kh = (lane >> 5) * 8;
-    const uint16_t* wsrc = W + (size_t)(tid >> 1) * K + (tid & 1) * 8;
-    uint4 c0, c1;
-    __builtin_memcpy(&c0, wsrc, 16);
-    __builtin_memcpy(&c1, wsrc + 16, 16);
-    f32x16 acc[NT];  // seeded with the bias of the lane's output column, as in strip_layer
+// 64 outputs of a layer over the wave's rows, from the weight piece in `w`,
+// onto the biases in acc; meanwhile the next piece is fetched, the piece
+// before (`other`, if PREV) is finished into yprev, and its accumulators start
+// at the next piece's biases (if NEXT).  The 32x32x16 operands: lane l
+// holds A[l % 32][8 (l / 32) + v] and B[8 (l / 32) + v][l % 32], v < 8;
+// accumulator register r of lane l is D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
+// So the lane of row j holds outputs 4 h .. 4 h + 3 of every eight (h = l / 32),
+// and a swap of halves between the eights 2 i and 2 i + 1 gives each half all of
+// its eight.
+//
+// Two input steps (four products, 128 cycles) at a time: their weights were
+// read from LDS during the two before, and between the products, which leave
+// seven in eight issue slots free, go the reads for the next two, a step of the
+// fetch and a quarter of the piece before.
+template <int KS, bool PREV, bool NEXT, typename F>
+__device__ __forceinline__ void piece(const bf16x8* x, PieceAcc& acc, PieceAcc& other, bf16x8* yprev, const uint4* w,
+                                      const float* next_bias, const F& fetch) {
+    constexpr int kPairs = (KS + 1) / 2;
+    constexpr int kValu = 0x2, kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100;
+    static_assert(kPairs >= 4, "a quarter of the piece before in each of four pairs");
+    static_assert(kPieceTiles == 2, "four products in a pair");
+    bf16x8 a[2][4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = (f32x16)(bias[t * 32 + row]);
-    const uint16_t* a_row = io + row * kLdsStride + kh;
-    // unrolled so that the two chunks in flight swap registers instead of
-    // being copied each step (four steps measured faster than two)
-#pragma unroll 4
-    for (int ks = 0; ks < KS; ++ks) {
-        __syncthreads();  // the previous chunk has been read
-        __builtin_memcpy(s_w + tid * 8, &c0, 16);
-        c0 = c1;
-        if (ks + 2 < KS) __builtin_memcpy(&c1, wsrc + (ks + 2) * 16, 16);
-        __syncthreads();
-        if (active) {
-            const bf16x8 a = load8(a_row + ks * 16);
+    for (int j = 0; j < 4; ++j) a[0][j] = weight_operand<KS>(w, j % 2, j / 2);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const bf16x8 b = load8(s_w + (t * 32 + row) * 16 + kh);
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[t], 0, 0, 0);
-            }
+    for (int c = 0; c < kPairs; ++c) {
+        if (c + 1 < kPairs) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (2 * (c + 1) + j / 2 < KS) a[(c + 1) % 2][j] = weight_operand<KS>(w, j % 2, 2 * (c + 1) + j / 2);
         }
-    }
-    if (!active) return;
-    // Rows rr and rr + 1 of column c are converted together; each even lane
-    // then swaps halves with the odd lane beside it (column c + 1), so that
-    // the even lane stores row rr and the odd lane row rr + 1 of the column
-    // pair (c & ~1, c | 1) as one 32-bit word.
-    const int r0 = (lane >> 5) * 4;
-    const bool odd = lane & 1;
-    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;  // bytes of (neighbour, own)
+        fetch.step(c);
+        if (c + 1 == kPairs && F::kSteps > kPairs) fetch.step(kPairs);
+        if (PREV && c < 4) yprev[c] = finish_quarter(other, c);
+        if (NEXT && c + 1 == kPairs) start_piece(other, next_bias);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int c = t * 32 + (row & ~1);
+        for (int j = 0; j < 4; ++j)
+            if (2 * c + j / 2 < KS)
+                acc[j % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[c % 2][j], x[2 * c + j / 2], acc[j % 2], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            const int rr = (r >> 2) * 8 + r0 + (r & 3) + (odd ? 1 : 0);
-            const uint32_t p = pack_bf16(lrelu(acc[t][r]), lrelu(acc[t][r + 1]));
-            const uint32_t q = (uint32_t)__builtin_amdgcn_mov_dpp((int)p, 0xB1, 0xF, 0xF, false);
-            *reinterpret_cast<uint32_t*>(io + rr * kLdsStride + c) = __builtin_amdgcn_perm(q, p, sel);
+        for (int j = 1; j < 4; ++j) {
+            __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kValu, 6, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
+}
+
+// A layer of 64 NP outputs over operands x[KS].  Its first piece's copy into
+// w0 is under way and its biases are in acc0; each piece is multiplied while
+// the next one's copy (after the last piece: the following layer's first, with
+// NKS steps and as many outputs, if NKS) fills the other buffer, and while the
+// piece before is finished: before this layer's first, the last of the layer
+// before (its four operands x[XL ..], if XL >= 0).  NP is even, so that every
+// layer starts at w0 and acc0; its last piece stays in acc1.  s_bias: of this
+// layer, the following one's after it.  Every wave of the block calls it.
+template <int KS, int NP, int NKS, int XL, bool ALIGNED, int P = 0>
+__device__ __forceinline__ void layer(bf16x8* x, bf16x8* y, PieceAcc& acc0, PieceAcc& acc1, uint4* w0, uint4* w1,
+                                      const uint16_t* W, const uint16_t* Wnext, const float* s_bias) {
+    static_assert(NP % 2 == 0, "the next layer starts at w0");
+    __syncthreads();  // this piece is there, and the other buffer has been read
+    constexpr bool kSame = P + 1 < NP;
+    using F = std::conditional_t<kSame, Fetch<KS, kPiece * NP, ALIGNED>,
+                                 std::conditional_t<(NKS > 0), Fetch<NKS, kPiece * NP, ALIGNED>, NoFetch>>;
+    const F fetch(kSame ? W : Wnext, kSame ? kPiece * (P + 1) : 0, P % 2 ? w0 : w1);
+    constexpr bool kNext = P + 1 < NP || NKS > 0;
+    const float* next_bias = s_bias + kPiece * (P + 1);
+    if constexpr (P % 2 != 0) piece<KS, true, kNext>(x, acc1, acc0, y + 4 * (P - 1), w1, next_bias, fetch);
+    else if constexpr (P > 0) piece<KS, true, kNext>(x, acc0, acc1, y + 4 * (P - 1), w0, next_bias, fetch);
+    else piece<KS, (XL >= 0), kNext>(x, acc0, acc1, x + (XL >= 0 ? XL : 0), w0, next_bias, fetch);
+    if constexpr (P + 1 < NP)
+        layer<KS, NP, NKS, XL, ALIGNED, P + 1>(x, y, acc0, acc1, w0, w1, W, Wnext, s_bias);
 }
 
 struct PairArgs {
@@ -244,59 +308,80 @@ struct PairArgs {
     const uint8_t* valid;  // [M, K]
     const float* rays_d;   // [M, 3]
     int64_t M;
-    int K, kp_log2;
+    int K, ns;             // ns: samples of a block
     epcq_aggregator_params p;
     float* out_alpha;      // [M]
-    uint16_t* xc;          // [M, 288] bf16 colour-branch inputs
+    uint16_t* xc;          // [M, 256] bf16 sums of the pairs' features
 };
 
-__global__ __launch_bounds__(kPairBlock) void agg_pair_kernel(PairArgs a) {
-    __shared__ __align__(16) uint16_t s_rows[kPairWaves][kStrip * kLdsStride];
-    __shared__ __align__(16) uint16_t s_w[kH * 16];
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    uint16_t* io = s_rows[wave];
-    const int Kp = 1 << a.kp_log2;
-    const int64_t rows_total = (int64_t)a.M << a.kp_log2;
-    if ((int64_t)blockIdx.x * kPairWaves * kStrip >= rows_total) return;  // whole block past the end
-    const int64_t row0 = ((int64_t)blockIdx.x * kPairWaves + wave) * kStrip;
-    const bool live_strip = row0 < rows_total;  // waves past the end still take part in the copies
+template <bool ALIGNED>
+__global__ __launch_bounds__(kBlock, 2) void agg_pair_kernel(PairArgs a) {
+    // two arrays, so that reading one needs no wait for the copies to the other
+    __shared__ uint4 s_w0[kPieceBytes / 16];
+    __shared__ uint4 s_w1[kPieceBytes / 16];
+    __shared__ __align__(16) float s_bias[4 * kH];
+    __shared__ __align__(16) float s_wa[kH];
+    __shared__ float s_inv[kRows], s_alpha[kRows];
+    const uint16_t* w1 = static_cast<const uint16_t*>(a.p.w1);
+    const uint16_t* w2 = static_cast<const uint16_t*>(a.p.w2);
+    const uint16_t* w3 = static_cast<const uint16_t*>(a.p.w3);
+    const uint16_t* w4 = static_cast<const uint16_t*>(a.p.w4);
+    const int tid = threadIdx.x;
+    const int wave = tid / kWave;
+    const int lane = tid % kWave;
     const int row = lane & 31;
     const int half = lane >> 5;
-    const int64_t r = row0 + row;
-    const int64_t m = r >> a.kp_log2;
-    const int k = (int)(r & (Kp - 1));
-    const bool in_range = m < a.M;
-    const bool valid = in_range && k < a.K && a.valid[m * a.K + k] != 0;
-    const int64_t pair = m * a.K + k;
+    const int brow = wave * kWaveRows + row;  // row of the block
+    const int64_t m0 = (int64_t)blockIdx.x * a.ns;
+    const int s = brow / a.K;
+    const int64_t m = m0 + s;
+    const bool in_range = s < a.ns && m < a.M;
+    const int64_t pair = m0 * a.K + brow;
 
-    // ---- x1 rows: lane half 0 takes features 0..15, half 1 features 16..31
-    // and the distance terms; invalid rows are zero
+    // ---- the rows' inputs: each lane half takes every other four features.
+    // The loads of all rows are under way together, before the weights'; an
+    // invalid pair's values are dropped afterwards.
+    bool valid = false;
     float px = 0.0f, py = 0.0f, pz = 0.0f, sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    float rgb[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f}, rd[3] = {0.0f, 0.0f, 0.0f};
+    float4 fv[4] = {};
     if (in_range) {
-        sx = a.sp_xyz[3 * m];
-        sy = a.sp_xyz[3 * m + 1];
-        sz = a.sp_xyz[3 * m + 2];
-    }
-    if (valid) {
+        valid = a.valid[pair] != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fv[i] = reinterpret_cast<const float4*>(a.pc_feat + pair * kFeat)[2 * i + half];
         px = a.pc_xyz[3 * pair];
         py = a.pc_xyz[3 * pair + 1];
         pz = a.pc_xyz[3 * pair + 2];
-    }
-    uint16_t* xr = io + row * kLdsStride;
-    float4 fv[4];
+        sx = a.sp_xyz[3 * m];
+        sy = a.sp_xyz[3 * m + 1];
+        sz = a.sp_xyz[3 * m + 2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        fv[q] = valid ? reinterpret_cast<const float4*>(a.pc_feat + pair * kFeat + half * 16)[q]
-                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int i = 0; i < 3; ++i) {
+            rgb[i] = a.pc_rgb[3 * pair + i];
+            dir[i] = a.pc_dir[3 * pair + i];
+            rd[i] = a.rays_d[3 * m + i];
+        }
+    }
+    Fetch<kX1 / 16, kH, ALIGNED>(w1, 0, s_w0).all();
+    s_bias[tid] = a.p.b1[tid];
+    s_bias[kH + tid] = a.p.b2[tid];
+    s_bias[2 * kH + tid] = a.p.b3[tid];
+    s_bias[3 * kH + tid] = a.p.b4[tid];
+    s_wa[tid] = a.p.wa[tid];
+    if (!valid) {
+        px = py = pz = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fv[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) rgb[i] = dir[i] = 0.0f;
+    }
+    // ---- x1, as operands
     const float* fs = reinterpret_cast<const float*>(fv);
-    {
-        uint4 w0 = make_uint4(pack_bf16(fs[0], fs[1]), pack_bf16(fs[2], fs[3]), pack_bf16(fs[4], fs[5]),
-                              pack_bf16(fs[6], fs[7]));
-        uint4 w1 = make_uint4(pack_bf16(fs[8], fs[9]), pack_bf16(fs[10], fs[11]), pack_bf16(fs[12], fs[13]),
-                              pack_bf16(fs[14], fs[15]));
-        __builtin_memcpy(xr + half * 16, &w0, 16);
-        __builtin_memcpy(xr + half * 16 + 8, &w1, 16);
+    bf16x8 x[kX1 / 16], y[kX3 / 16];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float* f = fs + 8 * i;
+        x[i] = swap_halves(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7]));
     }
     // dist = p - s and distpow = p^2 - s^2; invalid pairs have p = 0 as the
     // reference's zero-filled gathers
@@ -304,33 +389,56 @@ __global__ __launch_bounds__(kPairBlock) void agg_pair_kernel(PairArgs a) {
     auto encode = [&](auto checked) {
         constexpr bool C = decltype(checked)::value;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            // PE(f, 3) of feature d = half * 16 + i: 6 values at 32 + 6 d
-            float sn[3], cs[3];
-            pe_sincos<C>(fs[i], sn[0], cs[0]);
-            pe_double(sn[0], cs[0], sn[1], cs[1]);
-            pe_double(sn[1], cs[1], sn[2], cs[2]);
-            uint32_t* o = reinterpret_cast<uint32_t*>(xr + kFeat + 6 * (half * 16 + i));
-            o[0] = pack_bf16(sn[0], cs[0]);
-            o[1] = pack_bf16(sn[1], cs[1]);
-            o[2] = pack_bf16(sn[2], cs[2]);
-        }
-        if (half) {
-            uint32_t* o = reinterpret_cast<uint32_t*>(xr + 224);
+        for (int i = 0; i < 4; ++i) {
+            // PE(f, 3): the lane's four features give 24 columns, three eights;
+            // those of half 0 and half 1 follow each other
+            uint32_t e[12];
 #pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                // frequencies 1 and 4 directly; 2, 8 and 16 by doubling
-                float sn[5], cs[5];
-                pe_sincos<C>(df[i], sn[0], cs[0]);
-                pe_sincos<C>(df[i] * 4.0f, sn[2], cs[2]);
+            for (int j = 0; j < 4; ++j) {
+                float sn[3], cs[3];
+                pe_sincos<C>(fs[4 * i + j], sn[0], cs[0]);
                 pe_double(sn[0], cs[0], sn[1], cs[1]);
-                pe_double(sn[2], cs[2], sn[3], cs[3]);
-                pe_double(sn[3], cs[3], sn[4], cs[4]);
+                pe_double(sn[1], cs[1], sn[2], cs[2]);
 #pragma unroll
-                for (int j = 0; j < 5; ++j) o[i * 5 + j] = pack_bf16(sn[j], cs[j]);
+                for (int q = 0; q < 3; ++q) e[3 * j + q] = pack_bf16(sn[q], cs[q]);
             }
-            o[30] = 0;  // columns 284..287
-            o[31] = 0;
+            // the six eights B0 B1 B2 (half 0), C0 C1 C2 (half 1) as operands
+            // (B0 | B1), (B2 | C0), (C1 | C2): the middle one is in place, and
+            // one swap of (B0 | C1) with (B1 | C2) gives the others
+            uint32_t lo[4], mid[4], hi[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t d0 = half ? e[4 + q] : e[q];
+                const uint32_t d1 = half ? e[8 + q] : e[4 + q];
+                mid[q] = half ? e[q] : e[8 + q];
+                const auto sw = __builtin_amdgcn_permlane32_swap(d0, d1, false, false);
+                lo[q] = sw[0];
+                hi[q] = sw[1];
+            }
+            x[2 + 3 * i] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+            x[3 + 3 * i] = __builtin_bit_cast(bf16x8, make_uint4(mid[0], mid[1], mid[2], mid[3]));
+            x[4 + 3 * i] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+        }
+        uint32_t e[32];
+        e[30] = 0;  // columns 284..287
+        e[31] = 0;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            // frequencies 1 and 4 directly; 2, 8 and 16 by doubling
+            float sn[5], cs[5];
+            pe_sincos<C>(df[i], sn[0], cs[0]);
+            pe_sincos<C>(df[i] * 4.0f, sn[2], cs[2]);
+            pe_double(sn[0], cs[0], sn[1], cs[1]);
+            pe_double(sn[2], cs[2], sn[3], cs[3]);
+            pe_double(sn[3], cs[3], sn[4], cs[4]);
+#pragma unroll
+            for (int j = 0; j < 5; ++j) e[i * 5 + j] = pack_bf16(sn[j], cs[j]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t* l = e + 8 * i;
+            x[14 + i] = __builtin_bit_cast(bf16x8, half ? make_uint4(l[4], l[5], l[6], l[7])
+                                                        : make_uint4(l[0], l[1], l[2], l[3]));
         }
     };
     // one test for the wave: when every argument of its encodings is below
@@ -339,168 +447,169 @@ __global__ __launch_bounds__(kPairBlock) void agg_pair_kernel(PairArgs a) {
     bool large = false;
 #pragma unroll
     for (int i = 0; i < 16; ++i) large = large || !(fabsf(fs[i]) < 1024.0f);
-    if (half) {
 #pragma unroll
-        for (int i = 0; i < 6; ++i) large = large || !(fabsf(df[i] * 4.0f) < 1024.0f);
-    }
+    for (int i = 0; i < 6; ++i) large = large || !(fabsf(df[i] * 4.0f) < 1024.0f);
     if (__ballot(large) == 0) encode(std::false_type{});
     else encode(std::true_type{});
-    const bool any_valid = __ballot(valid) != 0;
-    block_layer<kX1 / 16>(io, s_w, static_cast<const uint16_t*>(a.p.w1), a.p.b1, any_valid);
-    block_layer<kH / 16>(io, s_w, static_cast<const uint16_t*>(a.p.w2), a.p.b2, any_valid);
-    if (any_valid) {
-        // x3 = [h2, rgb, dir - d, dir . d, 0...]
-        if (half == 0) {
-            float rgb[3] = {0.0f, 0.0f, 0.0f}, dir[3] = {0.0f, 0.0f, 0.0f}, rd[3] = {0.0f, 0.0f, 0.0f};
-            if (valid) {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    rgb[i] = a.pc_rgb[3 * pair + i];
-                    dir[i] = a.pc_dir[3 * pair + i];
-                }
-            }
-            if (in_range) {
-#pragma unroll
-                for (int i = 0; i < 3; ++i) rd[i] = a.rays_d[3 * m + i];
-            }
-            float dot = dir[0] * rd[0];
-            dot = dot + dir[1] * rd[1];
-            dot = dot + dir[2] * rd[2];
-            xr[kH + 0] = to_bf16(rgb[0]);
-            xr[kH + 1] = to_bf16(rgb[1]);
-            xr[kH + 2] = to_bf16(rgb[2]);
-            xr[kH + 3] = to_bf16(dir[0] - rd[0]);
-            xr[kH + 4] = to_bf16(dir[1] - rd[1]);
-            xr[kH + 5] = to_bf16(dir[2] - rd[2]);
-            xr[kH + 6] = to_bf16(dot);
-        } else {
-#pragma unroll
-            for (int c = kH + 7; c < kX3; ++c) xr[c] = 0;
-        }
+    // x3 = [h2, rgb, dir - d, dir . d, 0...]: its last operand
+    float dot = dir[0] * rd[0];
+    dot = dot + dir[1] * rd[1];
+    dot = dot + dir[2] * rd[2];
+    const uint4 tail = half ? make_uint4(0, 0, 0, 0)
+                            : make_uint4(pack_bf16(rgb[0], rgb[1]), pack_bf16(rgb[2], dir[0] - rd[0]),
+                                         pack_bf16(dir[1] - rd[1], dir[2] - rd[2]), pack_bf16(dot, 0.0f));
+    if (__syncthreads_or(valid)) {  // the biases are there; blocks without a valid pair skip the layers
+        PieceAcc acc0, acc1;
+        start_piece(acc0, s_bias);
+        constexpr int kLast = kH / 16 - 4;  // operands of a layer's last piece
+        layer<kX1 / 16, 4, kH / 16, -1, ALIGNED>(x, y, acc0, acc1, s_w0, s_w1, w1, w2, s_bias);
+        layer<kH / 16, 4, kX3 / 16, kLast, ALIGNED>(y, x, acc0, acc1, s_w0, s_w1, w2, w3, s_bias + kH);
+        x[kH / 16] = __builtin_bit_cast(bf16x8, tail);
+        layer<kX3 / 16, 4, kH / 16, kLast, ALIGNED>(x, y, acc0, acc1, s_w0, s_w1, w3, w4, s_bias + 2 * kH);
+        layer<kH / 16, 4, 0, kLast, ALIGNED>(y, x, acc0, acc1, s_w0, s_w1, w4, nullptr, s_bias + 3 * kH);
+        finish_piece(acc1, x + kLast);
     }
-    block_layer<kX3 / 16>(io, s_w, static_cast<const uint16_t*>(a.p.w3), a.p.b3, any_valid);
-    block_layer<kH / 16>(io, s_w, static_cast<const uint16_t*>(a.p.w4), a.p.b4, any_valid);
-    if (!live_strip) return;
-    if (!any_valid)
-        for (int c = half * 128; c < half * 128 + 128; ++c) xr[c] = 0;
+    __syncthreads();  // every wave has read its weights: the buffers take the rows
 
-    // ---- per-pair alpha: lane halves take 128 columns each
-    float part = 0.0f;
-    {
-        const float4* wa4 = reinterpret_cast<const float4*>(a.p.wa + half * 128);
-        const uint16_t* hr = xr + half * 128;
-#pragma unroll 8
-        for (int q = 0; q < 32; ++q) {
-            const float4 wq = wa4[q];
-            uint2 h;
-            __builtin_memcpy(&h, hr + 4 * q, sizeof(h));
-            // fused multiply-adds (one rounding each; the module's fp32 sums are
-            // matched within the bf16 tolerance either way)
-            part = __builtin_fmaf(wq.x, __uint_as_float(h.x << 16), part);
-            part = __builtin_fmaf(wq.y, __uint_as_float(h.x & 0xffff0000u), part);
-            part = __builtin_fmaf(wq.z, __uint_as_float(h.y << 16), part);
-            part = __builtin_fmaf(wq.w, __uint_as_float(h.y & 0xffff0000u), part);
-        }
+    auto lds_row = [&](int r) {
+        uint16_t* base = reinterpret_cast<uint16_t*>(r < 2 * kWaveRows ? s_w0 : s_w1);
+        return base + (r % (2 * kWaveRows)) * kLdsStride;
+    };
+    // ---- the rows for the reductions; an invalid pair's is zero
+    uint16_t* xr = lds_row(brow);
+    if (valid) {
+#pragma unroll
+        for (int i = 0; i < kH / 16; ++i) *reinterpret_cast<bf16x8*>(xr + 16 * i + 8 * half) = x[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < kH / 16; ++i) *reinterpret_cast<bf16x8*>(xr + 16 * i + 8 * half) = bf16x8{};
     }
-    const float other = __shfl_xor(part, 32);
-    const float dotv = (half ? other + part : part + other) + a.p.ba[0];
-    const float alpha_k = softplus(dotv - 1.0f);
-
-    // ---- inverse-distance weights of the strip's samples (rows of a sample
-    // are lanes [s Kp, s Kp + Kp) of each half)
-    float dx = px - sx, dy = py - sy, dz = pz - sz;
+    // ---- per-pair alpha, each lane half over the columns that it holds
+    // (fused multiply-adds: one rounding each)
+    float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < kH / 16; ++i) {
+        const uint4 h = __builtin_bit_cast(uint4, x[i]);
+        const float4 wl = *reinterpret_cast<const float4*>(s_wa + 16 * i + 8 * half);
+        const float4 wh = *reinterpret_cast<const float4*>(s_wa + 16 * i + 8 * half + 4);
+        part[0] = __builtin_fmaf(wl.x, __uint_as_float(h.x << 16), part[0]);
+        part[1] = __builtin_fmaf(wl.y, __uint_as_float(h.x & 0xffff0000u), part[1]);
+        part[2] = __builtin_fmaf(wl.z, __uint_as_float(h.y << 16), part[2]);
+        part[3] = __builtin_fmaf(wl.w, __uint_as_float(h.y & 0xffff0000u), part[3]);
+        part[0] = __builtin_fmaf(wh.x, __uint_as_float(h.z << 16), part[0]);
+        part[1] = __builtin_fmaf(wh.y, __uint_as_float(h.z & 0xffff0000u), part[1]);
+        part[2] = __builtin_fmaf(wh.z, __uint_as_float(h.w << 16), part[2]);
+        part[3] = __builtin_fmaf(wh.w, __uint_as_float(h.w & 0xffff0000u), part[3]);
+    }
+    const float sum4 = (part[0] + part[1]) + (part[2] + part[3]);
+    const float dotv = sum4 + __shfl_xor(sum4, 32) + a.p.ba[0];
+    // ---- inverse distances, for the weights
+    const float dx = px - sx, dy = py - sy, dz = pz - sz;
     float nrm = dx * dx;
     nrm = nrm + dy * dy;
     nrm = nrm + dz * dz;
-    const float inv = valid ? 1.0f / (sqrtf(nrm) + 1e-6f) : 0.0f;
-    const int base = (row & ~(Kp - 1)) + half * 32;
-    float sum = 0.0f;
-    for (int j = 0; j < Kp; ++j) sum += __shfl(inv, base + j);
-    const float w = inv / (sum + 1e-6f);
+    if (half == 0) {
+        s_inv[brow] = valid ? 1.0f / (sqrtf(nrm) + 1e-6f) : 0.0f;
+        s_alpha[brow] = valid ? softplus(dotv - 1.0f) : 0.0f;
+    }
+    __syncthreads();
 
-    // ---- per sample: alpha, weighted feature sum and PE(d, 4) -> xc row
-    const int ns = kStrip >> a.kp_log2;
-    for (int s = 0; s < ns; ++s) {
-        const int64_t ms = (row0 >> a.kp_log2) + s;
+    // ---- per sample, one for each half of the wave and eight columns for each
+    // lane: weights, alpha and the weighted feature sum, in the order of the
+    // neighbours
+    for (int i = 2 * wave + half; i < a.ns && m0 + i < a.M; i += 2 * kWaves) {
+        const int r0 = i * a.K;
+        float sum = 0.0f;
+        for (int j = 0; j < a.K; ++j) sum += s_inv[r0 + j];
+        sum += 1e-6f;
         float acc_a = 0.0f;
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int j = 0; j < Kp; ++j) {
-            // every lane reads the same source row (a wave-uniform lane), so
-            // the values come from registers by readlane, with no LDS round
-            // trip, and the branch is uniform
-            const int src = s * Kp + j;
-            const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), src));
-            const float aj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(alpha_k), src));
-            const int vj = __builtin_amdgcn_readlane((int)valid, src);
-            if (!vj) continue;
-            acc_a = __builtin_fmaf(wj, aj, acc_a);
-            uint2 h;
-            __builtin_memcpy(&h, io + src * kLdsStride + lane * 4, sizeof(h));
-            acc[0] = __builtin_fmaf(wj, __uint_as_float(h.x << 16), acc[0]);
-            acc[1] = __builtin_fmaf(wj, __uint_as_float(h.x & 0xffff0000u), acc[1]);
-            acc[2] = __builtin_fmaf(wj, __uint_as_float(h.y << 16), acc[2]);
-            acc[3] = __builtin_fmaf(wj, __uint_as_float(h.y & 0xffff0000u), acc[3]);
+        float acc[8] = {};
+        for (int j = 0; j < a.K; ++j) {
+            const float wj = s_inv[r0 + j] / sum;
+            acc_a = __builtin_fmaf(wj, s_alpha[r0 + j], acc_a);
+            const uint4 h = *reinterpret_cast<const uint4*>(lds_row(r0 + j) + row * 8);
+            const uint32_t hw[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                acc[2 * q] = __builtin_fmaf(wj, __uint_as_float(hw[q] << 16), acc[2 * q]);
+                acc[2 * q + 1] = __builtin_fmaf(wj, __uint_as_float(hw[q] & 0xffff0000u), acc[2 * q + 1]);
+            }
         }
-        if (ms >= a.M) continue;
-        uint16_t* xo = a.xc + ms * kXc;
-        const uint2 packed = make_uint2((uint32_t)to_bf16(acc[0]) | ((uint32_t)to_bf16(acc[1]) << 16),
-                                        (uint32_t)to_bf16(acc[2]) | ((uint32_t)to_bf16(acc[3]) << 16));
-        __builtin_memcpy(xo + lane * 4, &packed, sizeof(packed));
-        if (lane < 12) {
-            const int i = lane / 4, j = lane % 4;
-            float sn, cs;
-            pe_sincos(a.rays_d[3 * ms + i] * (float)(1 << j), sn, cs);
-            reinterpret_cast<uint32_t*>(xo + kH)[lane] = pack_bf16(sn, cs);
-        } else if (lane < 20) {
-            xo[kH + 24 + (lane - 12)] = 0;
-        }
-        if (lane == 0) a.out_alpha[ms] = acc_a;
+        const uint4 packed = make_uint4(pack_bf16(acc[0], acc[1]), pack_bf16(acc[2], acc[3]),
+                                        pack_bf16(acc[4], acc[5]), pack_bf16(acc[6], acc[7]));
+        reinterpret_cast<uint4*>(a.xc + (m0 + i) * kH)[row] = packed;
+        if (row == 0) a.out_alpha[m0 + i] = acc_a;
     }
 }
 
 struct ColorArgs {
-    const uint16_t* xc;  // [M, 288]
+    const uint16_t* xc;  // [M, 256]
+    const float* rays_d; // [M, 3]
     int64_t M;
     epcq_aggregator_params p;
     float* out_rgb;      // [M, 3]
 };
 
-__global__ __launch_bounds__(kBlock) void agg_color_kernel(ColorArgs a) {
-    __shared__ __align__(16) uint16_t s_rows[kWavesPerBlock][kStrip * kLdsStride];
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x % kWave;
-    uint16_t* io = s_rows[wave];
-    const int64_t m0 = ((int64_t)blockIdx.x * kWavesPerBlock + wave) * kStrip;
-    if (m0 >= a.M) return;
-    const int row = lane & 31;
-    const int half = lane >> 5;
-    const int64_t m = m0 + row;
-    // stage the strip's inputs (rows past M are zero)
-    uint16_t* xr = io + row * kLdsStride;
-    for (int c = half * 8; c < kXc; c += 16) {
-        bf16x8 v = bf16x8{};
-        if (m < a.M) v = load8(a.xc + m * kXc + c);
-        __builtin_memcpy(xr + c, &v, sizeof(v));
+template <bool ALIGNED>
+__global__ __launch_bounds__(kBlock, 2) void agg_color_kernel(ColorArgs a) {
+    __shared__ uint4 s_w0[kPieceBytes / 16];
+    __shared__ uint4 s_w1[kPieceBytes / 16];
+    __shared__ __align__(16) float s_bias[3 * kC];
+    __shared__ __align__(16) float s_c4[3 * kC];
+    const uint16_t* c1 = static_cast<const uint16_t*>(a.p.c1);
+    const uint16_t* c2 = static_cast<const uint16_t*>(a.p.c2);
+    const uint16_t* c3 = static_cast<const uint16_t*>(a.p.c3);
+    Fetch<kXc / 16, kC, ALIGNED>(c1, 0, s_w0).all();
+    const int tid = threadIdx.x;
+    if (tid < kC) {
+        s_bias[tid] = a.p.cb1[tid];
+        s_bias[kC + tid] = a.p.cb2[tid];
+        s_bias[2 * kC + tid] = a.p.cb3[tid];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) s_c4[j * kC + tid] = a.p.c4[j * kC + tid];
     }
-    strip_layer<kXc / 16, kC / 32, true>(io, static_cast<const uint16_t*>(a.p.c1), a.p.cb1);
-    strip_layer<kC / 16, kC / 32, true>(io, static_cast<const uint16_t*>(a.p.c2), a.p.cb2);
-    strip_layer<kC / 16, kC / 32, true>(io, static_cast<const uint16_t*>(a.p.c3), a.p.cb3);
-    // last layer (128 -> 3) in fp32, halves take 64 columns each
+    const int lane = tid % kWave;
+    const int half = lane >> 5;
+    const int64_t m = (int64_t)blockIdx.x * kRows + tid / kWave * kWaveRows + (lane & 31);
+    bf16x8 x[kXc / 16], y[kC / 16];
+#pragma unroll
+    for (int i = 0; i < kH / 16; ++i) x[i] = m < a.M ? load8(a.xc + m * kH + 16 * i + 8 * half) : bf16x8{};
+    // PE(d, 4): half 0 takes d_x and d_z, half 1 d_y and the columns past it
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float d = m < a.M ? a.rays_d[3 * m + (i ? 2 : half)] : 0.0f;
+        uint32_t e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float sn, cs;
+            pe_sincos(d * (float)(1 << j), sn, cs);
+            e[j] = i && half ? 0 : pack_bf16(sn, cs);
+        }
+        x[kH / 16 + i] = __builtin_bit_cast(bf16x8, make_uint4(e[0], e[1], e[2], e[3]));
+    }
+    PieceAcc acc0, acc1;
+    __syncthreads();
+    start_piece(acc0, s_bias);
+    constexpr int kLast = kC / 16 - 4;
+    layer<kXc / 16, 2, kC / 16, -1, ALIGNED>(x, y, acc0, acc1, s_w0, s_w1, c1, c2, s_bias);
+    layer<kC / 16, 2, kC / 16, kLast, ALIGNED>(y, x, acc0, acc1, s_w0, s_w1, c2, c3, s_bias + kC);
+    layer<kC / 16, 2, 0, kLast, ALIGNED>(x, y, acc0, acc1, s_w0, s_w1, c3, nullptr, s_bias + 2 * kC);
+    finish_piece(acc1, y + kLast);
+    if (m >= a.M) return;
+    // last layer (128 -> 3) in fp32, each half the columns that it holds
     float part[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-    for (int q = 0; q < 16; ++q) {
-        const int c = half * 64 + 4 * q;
-        uint2 h;
-        __builtin_memcpy(&h, xr + c, sizeof(h));
-        const float hv[4] = {__uint_as_float(h.x << 16), __uint_as_float(h.x & 0xffff0000u),
-                             __uint_as_float(h.y << 16), __uint_as_float(h.y & 0xffff0000u)};
+#pragma unroll
+    for (int i = 0; i < kC / 16; ++i) {
+        const uint4 h = __builtin_bit_cast(uint4, y[i]);
+        const float hv[8] = {__uint_as_float(h.x << 16), __uint_as_float(h.x & 0xffff0000u),
+                             __uint_as_float(h.y << 16), __uint_as_float(h.y & 0xffff0000u),
+                             __uint_as_float(h.z << 16), __uint_as_float(h.z & 0xffff0000u),
+                             __uint_as_float(h.w << 16), __uint_as_float(h.w & 0xffff0000u)};
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const float4 wq = *reinterpret_cast<const float4*>(a.p.c4 + j * kC + c);
-            part[j] += wq.x * hv[0];
-            part[j] += wq.y * hv[1];
-            part[j] += wq.z * hv[2];
-            part[j] += wq.w * hv[3];
+            const float* wq = s_c4 + j * kC + 16 * i + 8 * half;
+#pragma unroll
+            for (int v = 0; v < 8; ++v) part[j] += wq[v] * hv[v];
         }
     }
 #pragma unroll
@@ -508,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void agg_color_kernel(ColorArgs a) {
         const float other = __shfl_xor(part[j], 32);
         const float v = (half ? other + part[j] : part[j] + other) + a.p.cb4[j];
         const float sig = 1.0f / (1.0f + expf(-v));
-        if (half == 0 && m < a.M) a.out_rgb[3 * m + j] = sig * (1.0f + 2.0f * 0.001f) - 0.001f;
+        if (half == 0) a.out_rgb[3 * m + j] = sig * (1.0f + 2.0f * 0.001f) - 0.001f;
     }
 }
 
@@ -519,7 +628,7 @@ using namespace epcq;
 
 extern "C" size_t epcq_aggregator_workspace_size(int64_t M) {
     if (M <= 0) return 0;
-    return (size_t)M * kXc * sizeof(uint16_t);
+    return (size_t)M * kH * sizeof(uint16_t);
 }
 
 extern "C" int epcq_aggregator_forward(const float* pc_xyz, const float* pc_rgb, const float* pc_dir,
@@ -548,21 +657,27 @@ extern "C" int epcq_aggregator_forward(const float* pc_xyz, const float* pc_rgb,
     pa.rays_d = rays_d;
     pa.M = M;
     pa.K = K;
-    pa.kp_log2 = ceil_log2(K);
+    pa.ns = kRows / K;
     pa.p = *params;
     pa.out_alpha = out_alpha;
     pa.xc = static_cast<uint16_t*>(workspace);
-    const int64_t strips = ceil_div(M << pa.kp_log2, kStrip);
-    const int64_t blocks = ceil_div(strips, kPairWaves);
+    const int64_t blocks = ceil_div(M, pa.ns);
     if (blocks > INT32_MAX) return fail(EPCQ_ERR_INVALID, "aggregator: too many samples");
-    agg_pair_kernel<<<dim3((unsigned)blocks), dim3(kPairBlock), 0, st>>>(pa);
+    uintptr_t low = 0;  // the load unit's copies to LDS want 16-byte alignment
+    for (const void* w : {params->w1, params->w2, params->w3, params->w4, params->c1, params->c2, params->c3})
+        low |= reinterpret_cast<uintptr_t>(w);
+    const bool aligned = (low & 15u) == 0;
+    if (aligned) agg_pair_kernel<true><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(pa);
+    else agg_pair_kernel<false><<<dim3((unsigned)blocks), dim3(kBlock), 0, st>>>(pa);
     if (int e = check_launch("aggregator/pairs")) return e;
     ColorArgs ca;
     ca.xc = pa.xc;
+    ca.rays_d = rays_d;
     ca.M = M;
     ca.p = *params;
     ca.out_rgb = out_rgb;
-    const int64_t cblocks = ceil_div(ceil_div(M, kStrip), kWavesPerBlock);
-    agg_color_kernel<<<dim3((unsigned)cblocks), dim3(kBlock), 0, st>>>(ca);
+    const dim3 cgrid((unsigned)ceil_div(M, kRows));
+    if (aligned) agg_color_kernel<true><<<cgrid, dim3(kBlock), 0, st>>>(ca);
+    else agg_color_kernel<false><<<cgrid, dim3(kBlock), 0, st>>>(ca);
     return check_launch("aggregator/colour");
 }
