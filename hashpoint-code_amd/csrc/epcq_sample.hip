@@ -133,8 +133,27 @@ __global__ __launch_bounds__(kBlock) void bucket_cone_kernel(const int2* __restr
     if (p < P) bucket_cone_body(hash, sorted_idx, xyz, pts_in, radius, r0, c2w, p, cone_a, cone_b, pts, prad);
 }
 
-// hashtable_query_for_nearby_point (:222-283): one lane per ray, hits of each
-// neighbour bucket (at most 32) appended in lane order.
+// Buckets of more points than this are taken one at a time, so that a group's
+// candidates are always counted in 31 bits.
+constexpr int kQueryBucket = 1 << 24;
+
+// Rays from which on windows of at most 32 buckets take half a wave per ray:
+// twice the rays per instruction, but with fewer rays whole waves fill the GPU
+// better (2513 rays of 1.4M points, 23 us, take one wave each).
+constexpr int64_t kQueryHalfWave = 16384;
+
+// hashtable_query_for_nearby_point (:222-283): hits of each neighbour bucket
+// (at most 32) appended in lane order.  G lanes take a ray: each reads the hash
+// entry of one bucket, a prefix sum numbers the candidates of G buckets, and
+// the lanes take G candidates at a time, whichever bucket they are in; a ballot
+// gives each hit its place in the output, so that reads of the list and writes
+// are consecutive.  With one lane per ray every candidate was a wait for
+// memory.  What bounds it now: instruction issue (about 250 per ray of 25
+// buckets) and the R * cap outputs.  Measured, one lane per ray against groups:
+// all 120k rays of 200k points at 400 x 300, cap 256 0.253 -> 0.050 ms; 1024
+// rays of 1M points at 200 x 160 1.97 -> 0.04; 480k rays of 2M points at 800 x
+// 600 1.33 -> 0.82; 500k rays of a nearly empty image 0.206 -> 0.122.
+template <int G>
 __global__ __launch_bounds__(kBlock) void query_kernel(const float* __restrict__ xyz,
                                                        const int* __restrict__ sorted_idx,
                                                        const int2* __restrict__ hash,
@@ -142,8 +161,12 @@ __global__ __launch_bounds__(kBlock) void query_kernel(const float* __restrict__
                                                        float cx, float cy, int W, int H, int k, int ko,
                                                        float r0, const int* __restrict__ rays, int64_t R,
                                                        int cap, int* __restrict__ out) {
-    const int64_t ri = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (ri >= R) return;
+    const int64_t ri = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / G;
+    if (ri >= R) return;  // whole groups
+    const int lane = threadIdx.x % G;
+    const int shift = threadIdx.x % kWave / G * G;  // the group's first lane in the wave
+    const uint64_t group = ~0ull >> (kWave - G);
+    const uint64_t below = (1ull << lane) - 1;  // of the group's ballots
     int* row = out + ri * cap;
     int total = 0;
     const int64_t q = rays[ri];
@@ -155,24 +178,63 @@ __global__ __launch_bounds__(kBlock) void query_kernel(const float* __restrict__
         Ray ray;
         make_ray(m, fx, fy, cx, cy, u, v, ray);
         const int L = k * k;
-        for (int l = 0; l < L && total < cap; ++l) {
-            const int2 e = hash[neighbor_pixel(k, ko, l, u, v, W, H)];
-            if (e.y < 0) continue;
-            int kept = 0;
-            for (int j = 0; j < e.y && kept < kQueryLaneHits; ++j) {
-                const int id = sorted_idx[e.x + j];
-                const float* p = xyz + 3 * (int64_t)id;
-                float t, dist;
-                point_ray(ray, p[0], p[1], p[2], t, dist);
-                if (dist < r0) {
-                    if (total < cap) row[total] = id;
-                    ++total;
-                    ++kept;
-                }
+        for (int l0 = 0; l0 < L && total < cap;) {
+            int2 e = make_int2(0, 0);
+            if (l0 + lane < L) e = hash[neighbor_pixel(k, ko, l0 + lane, u, v, W, H)];
+            int n = max(e.y, 0);
+            int step = G;
+            if ((__ballot(n > kQueryBucket) >> shift & group) != 0) {
+                step = 1;
+                if (lane != 0) n = 0;
             }
+            int end = n;  // candidates of the buckets up to the lane's
+#pragma unroll
+            for (int d = 1; d < G; d *= 2) {
+                const int t = __shfl_up(end, d, G);
+                if (lane >= d) end += t;
+            }
+            const int first = e.x - (end - n);  // list position of candidate c: first + c
+            const int C = __shfl(end, G - 1, G);
+            const bool capped = (__ballot(n > kQueryLaneHits) >> shift & group) != 0;
+            int carry = 0;  // hits so far of a bucket that began before c0
+            for (int c0 = 0; c0 < C && total < cap;) {
+                const int c = c0 + lane;
+                int b = 0;  // the candidate's bucket: the first that ends after it
+#pragma unroll
+                for (int d = G / 2; d > 0; d /= 2)
+                    if (__shfl(end, b + d - 1, G) <= c) b += d;
+                const int j = __shfl(first, b, G) + c;
+                bool hit = false;
+                int id = 0;
+                if (c < C) {
+                    id = sorted_idx[j];
+                    const float* p = xyz + 3 * (int64_t)id;
+                    float t, dist;
+                    point_ray(ray, p[0], p[1], p[2], t, dist);
+                    hit = dist < r0;
+                }
+                uint64_t mask = __ballot(hit) >> shift & group;
+                int next = c0 + G;
+                if (capped) {
+                    const int start = __shfl(end - n, b, G);
+                    const int s0 = max(start - c0, 0);  // the bucket's first lane
+                    const int before = __popcll(mask & below & (~0ull << s0)) + (start < c0 ? carry : 0);
+                    carry = __shfl(before + (hit ? 1 : 0), G - 1, G);
+                    // the rest of a bucket that is full
+                    const int stop = __shfl(end, __shfl(b, G - 1, G), G);
+                    if (carry >= kQueryLaneHits) next = max(next, stop);
+                    hit = hit && before < kQueryLaneHits;
+                    mask = __ballot(hit) >> shift & group;
+                }
+                const int at = total + __popcll(mask & below);
+                if (hit && at < cap) row[at] = id;
+                total += __popcll(mask);
+                c0 = next;
+            }
+            l0 += step;
         }
     }
-    for (int j = total; j < cap; ++j) row[j] = -1;
+    for (int j = total + lane; j < cap; j += G) row[j] = -1;
 }
 
 __global__ __launch_bounds__(kBlock) void idw_kernel(const float* __restrict__ xyz, const void* feat,
@@ -604,10 +666,14 @@ extern "C" int epcq_quick_query(const float* xyz, int64_t n, const epcq_camera* 
     if (R < 0) return fail(EPCQ_ERR_INVALID, "quick_query_for_nearby_point: negative ray count");
     (void)n;
     if (R == 0 || opt->num_point_per_ray == 0) return EPCQ_OK;
-    query_kernel<<<dim3((unsigned)ceil_div(R, kBlock)), dim3(kBlock), 0, as_stream(stream)>>>(
-        xyz, sorted_idx, reinterpret_cast<const int2*>(hash), cam->c2w, cam->fx, cam->fy, cam->cx, cam->cy,
-        cam->width, cam->height, opt->kernel_size, (opt->kernel_size + 1) / 2, opt->radius_threshold, rays, R,
-        opt->num_point_per_ray, out);
+    auto launch = [&](auto kernel, int lanes) {
+        kernel<<<dim3((unsigned)ceil_div(R, kBlock / lanes)), dim3(kBlock), 0, as_stream(stream)>>>(
+            xyz, sorted_idx, reinterpret_cast<const int2*>(hash), cam->c2w, cam->fx, cam->fy, cam->cx, cam->cy,
+            cam->width, cam->height, opt->kernel_size, (opt->kernel_size + 1) / 2, opt->radius_threshold, rays, R,
+            opt->num_point_per_ray, out);
+    };
+    if (k2 <= 32 && R >= kQueryHalfWave) launch(query_kernel<32>, 32);
+    else launch(query_kernel<64>, 64);
     return check_launch("quick_query_for_nearby_point");
 }
 
