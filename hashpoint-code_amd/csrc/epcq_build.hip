@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kBlock) void bin_scan_kernel(BuildView bv) {
 
 __global__ __launch_bounds__(kBlock) void build_bin_kernel(BuildView bv) {
     extern __shared__ int s_cur[];
-    bin_body(bv, blockIdx.x, s_cur);
+    bin_body(bv, xcd_tile((int)blockIdx.x, (int)gridDim.x), s_cur);
 }
 
 __global__ __launch_bounds__(kBlock) void build_fine_kernel(BuildView bv) {

@@ -20,6 +20,15 @@ constexpr int kMaxSlots = 128;       // MAX_SAMPLE_POINTS_NUM: depth slots per r
 
 constexpr int kWave = 64;
 
+// Maps block b of nb to a tile (or chunk) index so that the blocks the hardware
+// places on one XCD (b, b + 8, b + 16, ...) take consecutive ones and share halos
+// in that XCD's L2.
+__device__ __forceinline__ int xcd_tile(int b, int nb) {
+    const int per = nb / 8, rem = nb % 8;
+    const int x = b % 8, j = b / 8;
+    return x * per + min(x, rem) + j;
+}
+
 struct Ray {
     float o[3];
     float d[3];

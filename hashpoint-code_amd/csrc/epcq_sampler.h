@@ -1434,15 +1434,6 @@ __device__ __forceinline__ void run_ray_wave(const SampleOpts& o, const SampleOu
 // Smallest float s with sqrtf(s) >= r, so that sqrtf(e2) < r <=> e2 < s.
 float squared_threshold(float r);
 
-// Maps block b of nb to a tile index so that the blocks the hardware places
-// on one XCD (b, b + 8, b + 16, ...) take consecutive tiles and share halos
-// in that XCD's L2.
-__device__ __forceinline__ int xcd_tile(int b, int nb) {
-    const int per = nb / 8, rem = nb % 8;
-    const int x = b % 8, j = b / 8;
-    return x * per + min(x, rem) + j;
-}
-
 // Tile geometry of the LDS-staged sampler: a tw x th block of rays stages the
 // hash entries and points of its halo region (tw + k - 1) x (th + k - 1).
 struct TilePlan {
