@@ -228,7 +228,8 @@ int build_hashtable_impl(const float* xyz, int64_t n, const float* w2c, const fl
     if (height <= 0 || width <= 0) return fail(EPCQ_ERR_INVALID, w + ": image size must be positive");
     if (n < 0 || n >= (int64_t(1) << 31)) return fail(EPCQ_ERR_INVALID, w + ": point count out of range");
     if ((int64_t)height * width >= (int64_t(1) << 31) / 2) return fail(EPCQ_ERR_INVALID, w + ": image too large");
-    const BuildPlan bp = plan_build(n, height, width);
+    BuildPlan bp = plan_build(n, height, width);
+    if (workspace_bytes < bp.bytes) bp = plan_build(n, height, width, false, kBinPoints, false);
     if (workspace_bytes < bp.bytes || (bp.bytes && !workspace))
         return fail(EPCQ_ERR_WORKSPACE, w + ": workspace too small");
     hipStream_t st = as_stream(stream);
@@ -323,7 +324,7 @@ extern "C" int epcq_build_hashtable_noalloc(const float* xyz, int64_t n, const f
     const char* who = "build_hashtable_noalloc";
     if (height > 0 && width > 0 && n >= 0 && n < (int64_t(1) << 31) &&
         (int64_t)height * width < (int64_t(1) << 31) / 2) {
-        const size_t need = plan_build(n, height, width).bytes;
+        const size_t need = plan_build(n, height, width, false, kBinPoints, false).bytes;
         if (need > kNoallocScratchBytes)
             return fail(EPCQ_ERR_WORKSPACE, std::string(who) + ": needs " + std::to_string(need) +
                                                 " bytes of scratch, more than its " +

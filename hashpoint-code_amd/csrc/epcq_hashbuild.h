@@ -267,8 +267,12 @@ struct BuildView {
     int* part;    // [nseg][nbins]
     int* bstart;  // [nbins + 1]
     int* btotal;  // [nbins]
-    int4* trec;   // [n] binned (index, depth bits, pixel within bin, unused) records, or null (tpt)
-    float4* tpt;  // [n] binned (x, y, z, index bits) records, or null
+    // one of three binned forms, the others null:
+    float4* tpt;  // [n] (x, y, z, index bits) records
+    int4* trec;   // [n] (index, depth bits, pixel within bin, unused) records
+    int* tidx;    // [n] index, with tdep [n] and tfine [n], in a smaller workspace
+    float* tdep;
+    uint16_t* tfine;
     int* out_idx;     // [n]
     float* out_depth; // [n] (may be null: not written)
     int* out_hash;    // [P, 2]
@@ -284,20 +288,22 @@ struct BuildPlan {
     int64_t chunk;  // points per block in count / bin
     int nblk;
     int nseg;
-    size_t off_hist, off_part, off_start, off_total, off_rec, bytes;
-    bool points;
+    size_t off_hist, off_part, off_start, off_total, off_rec, off_tdep, off_tfine, bytes;
+    bool points, records;
 };
 
 // points: the bin pass carries each point's coordinates with its index (a
 // 16-byte record) so that the fine pass can write the pixel-ordered point
 // copy without gathering from xyz; no depth is binned then.  bin_points: the
 // points a bin of a dense view is sized to hold (the fine pass gives each bin
-// one block).
+// one block).  records false: the smaller workspace, 10 bytes per point instead
+// of 16, with index, depth and pixel in arrays of their own.
 // Largest block x bin count matrix the per-view build scans with one block
 // per bin (larger ones take the segmented scan).
 constexpr int64_t kColScanEntries = int64_t(1) << 20;
 
-inline BuildPlan plan_build(int64_t n, int H, int W, bool points = false, int bin_points = kBinPoints) {
+inline BuildPlan plan_build(int64_t n, int H, int W, bool points = false, int bin_points = kBinPoints,
+                            bool records = true) {
     BuildPlan bp{};
     bp.P = (int64_t)H * W;
     // bins of at most 2^kMaxTileShift pixels, fewer for dense views so that a
@@ -325,8 +331,11 @@ inline BuildPlan plan_build(int64_t n, int H, int W, bool points = false, int bi
     bp.off_part = take((size_t)bp.nseg * bp.nbins * 4);
     bp.off_start = take((size_t)(bp.nbins + 1) * 4);
     bp.off_total = take((size_t)bp.nbins * 4);
-    bp.off_rec = take((size_t)n * 16);
     bp.points = points;
+    bp.records = points || records;
+    bp.off_rec = take((size_t)n * (bp.records ? 16 : 4));
+    bp.off_tdep = take(bp.records ? 0 : (size_t)n * 4);
+    bp.off_tfine = take(bp.records ? 0 : (size_t)n * 2);
     bp.bytes = off;
     return bp;
 }
@@ -355,8 +364,15 @@ inline BuildView make_build_view(const BuildPlan& bp, const float* xyz, int64_t 
     v.part = reinterpret_cast<int*>(w + bp.off_part);
     v.bstart = reinterpret_cast<int*>(w + bp.off_start);
     v.btotal = reinterpret_cast<int*>(w + bp.off_total);
-    v.trec = bp.points ? nullptr : reinterpret_cast<int4*>(w + bp.off_rec);
-    v.tpt = bp.points ? reinterpret_cast<float4*>(w + bp.off_rec) : nullptr;
+    if (bp.points) {
+        v.tpt = reinterpret_cast<float4*>(w + bp.off_rec);
+    } else if (bp.records) {
+        v.trec = reinterpret_cast<int4*>(w + bp.off_rec);
+    } else {
+        v.tidx = reinterpret_cast<int*>(w + bp.off_rec);
+        v.tdep = reinterpret_cast<float*>(w + bp.off_tdep);
+        v.tfine = reinterpret_cast<uint16_t*>(w + bp.off_tfine);
+    }
     v.out_idx = out_idx;
     v.out_depth = out_depth;
     v.out_hash = out_hash;
@@ -499,8 +515,16 @@ __device__ __forceinline__ void bin_body(const BuildView& bv, int blk, int* s_cu
         const uint32_t bin = active ? ((uint32_t)key >> bv.ts) : 0u;
         const int pos = ordered_append(s_cur, bin, bv.bin_bits, active);
         if (active) {
-            if (bv.tpt) bv.tpt[pos] = make_float4(x, y, z, __int_as_float((int)i));
-            else bv.trec[pos] = make_int4((int)i, __float_as_int(depth), (int)((uint32_t)key & fmask), 0);
+            const uint32_t fine = (uint32_t)key & fmask;
+            if (bv.tpt) {
+                bv.tpt[pos] = make_float4(x, y, z, __int_as_float((int)i));
+            } else if (bv.trec) {
+                bv.trec[pos] = make_int4((int)i, __float_as_int(depth), (int)fine, 0);
+            } else {
+                bv.tidx[pos] = (int)i;
+                bv.tdep[pos] = depth;
+                bv.tfine[pos] = (uint16_t)fine;
+            }
         }
     }
     __syncthreads();
@@ -523,6 +547,10 @@ __device__ __forceinline__ void fine_body(const BuildView& bv, int b, int* s_mem
     if (bv.tpt) load_proj(bv.w2c, bv.K, bv.H, bv.W, pp);
     const uint32_t fmask = (uint32_t)tile - 1u;
     const float4* rec = bv.tpt ? bv.tpt : reinterpret_cast<const float4*>(bv.trec);
+    auto record = [&](int i) {
+        return rec ? rec[i]
+                   : make_float4(__int_as_float(bv.tidx[i]), bv.tdep[i], __int_as_float((int)bv.tfine[i]), 0.0f);
+    };
     auto fine_of = [&](const float4& q) -> uint32_t {
         if (!bv.tpt) return (uint32_t)__float_as_int(q.z);
         float depth;
@@ -531,7 +559,7 @@ __device__ __forceinline__ void fine_body(const BuildView& bv, int b, int* s_mem
     for (int f = threadIdx.x; f < tile; f += kBuildBlock) s_cnt[f] = 0;
     __syncthreads();
 #pragma unroll 4
-    for (int i = bs + threadIdx.x; i < bs + tot; i += kBuildBlock) atomicAdd(&s_cnt[fine_of(rec[i])], 1);
+    for (int i = bs + threadIdx.x; i < bs + tot; i += kBuildBlock) atomicAdd(&s_cnt[rec ? fine_of(rec[i]) : bv.tfine[i]], 1);
     __syncthreads();
     for (int f = threadIdx.x; f < tile; f += kBuildBlock) s_cur[f] = s_cnt[f];
     __syncthreads();
@@ -550,7 +578,7 @@ __device__ __forceinline__ void fine_body(const BuildView& bv, int b, int* s_mem
     // the next round's records load while this one's are placed
     float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     auto load = [&](int i) {
-        if (i < bs + tot) next = rec[i];
+        if (i < bs + tot) next = record(i);
     };
     load(bs + threadIdx.x);
     for (int r0 = bs; r0 < bs + tot; r0 += kBuildBlock) {
@@ -572,11 +600,13 @@ __device__ __forceinline__ void fine_body(const BuildView& bv, int b, int* s_mem
     }
     if (bv.sort && out_depth) {
         __syncthreads();
-        // each pixel run by depth; the records of this bin are free once placed
-        // and serve as the long runs' scratch (tot depths, then tot indices)
-        int* scratch = reinterpret_cast<int*>(bv.trec + bs) - bs;
-        sort_pixel_runs(tile, s_cnt, s_cur, bs, out_depth, bv.out_idx, reinterpret_cast<float*>(scratch),
-                        scratch + tot, s_wave);
+        // each pixel run by depth; what was binned is free once placed and
+        // serves as the long runs' scratch (records: tot depths, then tot
+        // indices)
+        int* scratch = bv.trec ? reinterpret_cast<int*>(bv.trec + bs) - bs : nullptr;
+        sort_pixel_runs(tile, s_cnt, s_cur, bs, out_depth, bv.out_idx,
+                        bv.trec ? reinterpret_cast<float*>(scratch) : bv.tdep, bv.trec ? scratch + tot : bv.tidx,
+                        s_wave);
     }
     // off-image tail: positions [N_in, n) hold -1 like the reference's
     // torch::full(-1) outputs; bin b fills every nbins-th run of 256

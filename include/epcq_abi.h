@@ -131,8 +131,9 @@ int epcq_scatter(const int32_t* point_idx, const int32_t* keys, const float* dep
  * scatter_hashtable).  xyz [n,3]; w2c >= 3 rows x 4 and K 3x3, row-major
  * device pointers.  Output as epcq_scatter_hashtable, with pixel lists
  * ordered by (pixel, point index), or (pixel, depth, point index) when
- * sort != 0.  workspace: device memory of at least
- * epcq_build_hashtable_workspace_size(n, height, width) bytes.
+ * sort != 0.  workspace: device memory of
+ * epcq_build_hashtable_workspace_size(n, height, width) bytes; one smaller by
+ * up to 6 bytes per point builds the same table more slowly.
  */
 size_t epcq_build_hashtable_workspace_size(int64_t n, int32_t height, int32_t width);
 int epcq_build_hashtable(const float* xyz, int64_t n, const float* w2c, const float* K,
@@ -146,8 +147,8 @@ int epcq_build_hashtable(const float* xyz, int64_t n, const float* w2c, const fl
  * serving loops, harnesses that forbid hipMalloc): epcq_build_hashtable with
  * its workspace in a device array the library holds, EPCQ_NOALLOC_SCRATCH_BYTES
  * on each GPU it runs on, for the life of the process.  Same outputs as
- * epcq_build_hashtable; returns EPCQ_ERR_WORKSPACE when
- * epcq_build_hashtable_workspace_size(n, height, width) exceeds that size.
+ * epcq_build_hashtable; returns EPCQ_ERR_WORKSPACE when the smallest workspace
+ * that epcq_build_hashtable takes for (n, height, width) exceeds that size.
  * It allocates nothing.  All calls on one GPU share its array: calls that
  * overlap on one GPU (different streams, or threads) race and must not be
  * made.
@@ -186,7 +187,8 @@ int epcq_quick_sampling_rays(const float* xyz, int64_t n, const epcq_camera* cam
 
 /* Workspace of the samplers for n points and an H x W image: per-pixel
  * bucket cones that let the walks skip neighbour pixels provably outside the
- * radius, and a pixel-ordered copy of the points.  Optional: with a NULL or
+ * radius, a pixel-ordered copy of the points, and a conservative bound of each
+ * point's reach in the image.  Optional: with a NULL or
  * smaller workspace the samplers skip nothing and gather the points through
  * sorted_idx (same results). */
 size_t epcq_sampling_workspace_size(int64_t n, int32_t height, int32_t width);
