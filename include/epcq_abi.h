@@ -79,8 +79,10 @@ const char* epcq_last_error(void);
  * wave (64 lanes share its candidate walks) after the tile's other rays,
  * instead of by one lane; 0 never does.  list_wave: a ray list (the rays
  * argument of the samplers) of at most this many rays is sampled one wave per
- * ray, longer ones one lane per ray; 0 never does.  Results are identical
- * either way.  Process-wide, guarded by a mutex; the autotuner sets it.
+ * ray, longer ones one lane per ray; 0 never does.  The row-run sampler, which
+ * takes most full images given a workspace, has tiles of its own and reads
+ * heavy as 8 to 32 times that many points.  Results are identical either way.
+ * Process-wide, guarded by a mutex; the autotuner sets it.
  * Defaults: 32, 8, 1024, 0, 128, 65536.
  */
 typedef struct epcq_tuning {
