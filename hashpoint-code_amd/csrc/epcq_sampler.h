@@ -1512,10 +1512,30 @@ __device__ __forceinline__ void tile_region(int W, int H, int k, int ko, int u0,
     RH = vz - va + 1;
 }
 
+// The list positions [lo, hi) from the first to the last of a row's n buckets
+// (0, 0 where all are empty).  False where a bucket begins before the one to
+// its left ends, as in a table whose buckets were moved or shared: such a row
+// is no run of the list, and staging [lo, hi) would read past the list and
+// index past the LDS.  Positions between two buckets (pixels taken out of the
+// table) are part of the run and are staged with it.
+__host__ __device__ __forceinline__ bool row_span(const int2* e, int n, int& lo, int& hi) {
+    lo = hi = 0;
+    bool found = false, ordered = true;
+    for (int c = 0; c < n; ++c) {
+        if (e[c].y <= 0) continue;
+        if (!found) lo = hi = e[c].x;
+        found = true;
+        ordered = ordered && e[c].x >= hi;
+        hi = e[c].x + e[c].y;
+    }
+    return ordered;
+}
+
 // Stages the halo region of the tile with top-left ray (u0, v0) into LDS:
 // its hash entries (rebased to the staged list), bucket cones (when
 // culling) and points.  Returns the number of staged points, or -1 if the
-// region holds more than `cap` points (the tile then reads global memory).
+// region holds more than `cap` points or a row of it is no run of the list
+// (the tile then reads global memory).
 // Block-wide; every thread of the block must call it.
 __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __restrict__ xyz,
                                           const float* __restrict__ radius, bool cull, int k, int ko, int u0, int v0,
@@ -1535,18 +1555,10 @@ __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __r
     }
     __syncthreads();
     for (int r = tid; r < RH; r += nthr) {
-        int lo = 0, hi = 0;
-        bool found = false;
-        for (int c = 0; c < RW; ++c) {
-            const int2 e = sm.hash[r * RW + c];
-            if (e.y > 0) {
-                if (!found) lo = e.x;
-                found = true;
-                hi = e.x + e.y;
-            }
-        }
+        int lo, hi;
+        const bool run = row_span(sm.hash + r * RW, RW, lo, hi);
         sm.rowlo[r] = lo;
-        sm.rowbase[r] = hi - lo;
+        sm.rowbase[r] = run ? hi - lo : INT_MAX;
     }
     __syncthreads();
     if (tid == 0) {
@@ -1554,7 +1566,7 @@ __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __r
         for (int r = 0; r < RH; ++r) {
             const int len = sm.rowbase[r];
             sm.rowbase[r] = run;
-            run += len;
+            run = len > cap - run ? cap + 1 : run + len;
         }
         sm.rowbase[RH] = run;
         *sm.total = run;
@@ -1570,13 +1582,12 @@ __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __r
             else hi = mid;
         }
         const int gi = sm.rowlo[lo] + (i - sm.rowbase[lo]);
-        int id;
+        // a position between two buckets may hold no index (-1), and its copy
+        // nothing: nobody reads what is staged for it
+        const int id = view.pts && (!radius || view.prad) ? 0 : max(view.sorted_idx[gi], 0);
         if (view.pts) {
-            const float4 q = view.pts[gi];
-            sm.pts[i] = q;
-            id = __float_as_int(q.w);
+            sm.pts[i] = view.pts[gi];
         } else {
-            id = view.sorted_idx[gi];
             const float* p = xyz + 3 * (int64_t)id;
             sm.pts[i] = make_float4(p[0], p[1], p[2], __int_as_float(id));
         }

@@ -167,6 +167,10 @@ int epcq_build_hashtable_noalloc(const float* xyz, int64_t n, const float* w2c, 
  * (bool bytes), S = num_sample_points_per_ray, Kc = num_point_cloud_per_sp.
  * For kernel_size > 5 (where the reference overflows its 32-entry neighbour
  * list) all kernel_size^2 neighbour pixels are used in both stages.
+ * sorted_idx and hash are any lists of this form, here and in the other
+ * samplers: each bucket lies inside the list and holds indices of points;
+ * buckets may be missing, in any order, or shared by pixels (rows that are not
+ * in the list's order are sampled more slowly).
  */
 int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camera* cam,
                         const epcq_options* opt, const int32_t* sorted_idx, const int32_t* hash,
