@@ -1,0 +1,47 @@
+"""Workspaces of the sizes that the library took before its 16-byte records and
+candidate bounds: the public calls take them and give the same outputs, bit for
+bit; what is smaller still is refused by the build."""
+import numpy as np
+import pytest
+import torch
+
+import epcq.csrc as C
+from epcq import synth
+from epcq.epcq import NeuralPoints, RenderOptions
+from scenes import bits, camera_spec, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def up(n):
+    return (n + 255) // 256 * 256
+
+
+def smallest_build(n, H, W):
+    """Index, depth and pixel in arrays of their own, in place of the records."""
+    return C.build_hashtable_workspace_size(n, H, W) - up(16 * n) + 2 * up(4 * n) + up(2 * n)
+
+
+def scene(n, W, H, dev):
+    cam = synth.look_at_camera([2.2, -2.4, 2.1], W, H, 1.39 * max(W, 48))
+    pts = synth.box_scene(max(n, 1000), n_boxes=12, seed=1)[:n]
+    return NeuralPoints(pc_type="pc", points=to_dev(np.ascontiguousarray(pts, np.float32), dev)), camera_spec(cam, dev)
+
+
+def same(a, b):
+    for x, y in zip(a, b):
+        assert np.array_equal(bits(x.cpu().numpy()), bits(y.cpu().numpy()))
+
+
+@pytest.mark.parametrize("sort", [False, True])
+@pytest.mark.parametrize("n,W,H", [(257, 9, 5), (60_000, 97, 65), (300_001, 640, 480)])
+def test_build_takes_ten_bytes_per_point(dev, n, W, H, sort):
+    npts, cs = scene(n, W, H, dev)
+    opt = RenderOptions()
+    small = smallest_build(n, H, W)
+    assert small < C.build_hashtable_workspace_size(n, H, W)
+    print("build workspace", n, W, H, sort, small, flush=True)
+    want = npts.pts2plane(cs, opt, sort=sort)
+    same(npts.pts2plane(cs, opt, sort=sort, workspace=torch.empty(small, dtype=torch.uint8, device=dev)), want)
+    with pytest.raises(RuntimeError, match="build_hashtable: workspace too small"):
+        npts.pts2plane(cs, opt, sort=sort, workspace=torch.empty(small - 1, dtype=torch.uint8, device=dev))
