@@ -229,7 +229,9 @@ int build_hashtable_impl(const float* xyz, int64_t n, const float* w2c, const fl
     if (n < 0 || n >= (int64_t(1) << 31)) return fail(EPCQ_ERR_INVALID, w + ": point count out of range");
     if ((int64_t)height * width >= (int64_t(1) << 31) / 2) return fail(EPCQ_ERR_INVALID, w + ": image too large");
     BuildPlan bp = plan_build(n, height, width);
-    if (workspace_bytes < bp.bytes) bp = plan_build(n, height, width, false, kBinPoints, false);
+    // the records want 16-byte alignment; index, depth and pixel of their own, four
+    if (workspace_bytes < bp.bytes || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        bp = plan_build(n, height, width, false, kBinPoints, false);
     if (workspace_bytes < bp.bytes || (bp.bytes && !workspace))
         return fail(EPCQ_ERR_WORKSPACE, w + ": workspace too small");
     hipStream_t st = as_stream(stream);

@@ -135,7 +135,8 @@ int epcq_scatter(const int32_t* point_idx, const int32_t* keys, const float* dep
  * ordered by (pixel, point index), or (pixel, depth, point index) when
  * sort != 0.  workspace: device memory of
  * epcq_build_hashtable_workspace_size(n, height, width) bytes; one smaller by
- * up to 6 bytes per point builds the same table more slowly.
+ * up to 6 bytes per point, or aligned to 4 bytes and not to 16, builds the same
+ * table more slowly.
  */
 size_t epcq_build_hashtable_workspace_size(int64_t n, int32_t height, int32_t width);
 int epcq_build_hashtable(const float* xyz, int64_t n, const float* w2c, const float* K,

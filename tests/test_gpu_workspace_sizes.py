@@ -45,3 +45,15 @@ def test_build_takes_ten_bytes_per_point(dev, n, W, H, sort):
     same(npts.pts2plane(cs, opt, sort=sort, workspace=torch.empty(small, dtype=torch.uint8, device=dev)), want)
     with pytest.raises(RuntimeError, match="build_hashtable: workspace too small"):
         npts.pts2plane(cs, opt, sort=sort, workspace=torch.empty(small - 1, dtype=torch.uint8, device=dev))
+
+
+@pytest.mark.parametrize("offset", [4, 8, 12])
+def test_build_takes_a_workspace_at_any_word(dev, offset):
+    n, W, H = 60_000, 97, 65
+    npts, cs = scene(n, W, H, dev)
+    opt = RenderOptions()
+    print("build workspace at", offset, flush=True)
+    for sort in (False, True):
+        for size in (smallest_build(n, H, W), C.build_hashtable_workspace_size(n, H, W)):
+            ws = torch.empty(offset + size, dtype=torch.uint8, device=dev)[offset:]
+            same(npts.pts2plane(cs, opt, sort=sort, workspace=ws), npts.pts2plane(cs, opt, sort=sort))
