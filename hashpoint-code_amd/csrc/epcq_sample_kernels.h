@@ -64,8 +64,8 @@ __global__ __launch_bounds__(kBlock) void sample_list_kernel(SampleOpts o, Sampl
     }
 }
 
-// One wave per listed ray (run_ray_wave, the same outputs as run_ray): for
-// short lists, such as a training batch, whose one-lane-per-ray form would
+// One wave per listed ray (run_ray_wave, the same outputs as run_ray), for
+// windows of at most 64 NW lanes: for short lists, such as a training batch, whose one-lane-per-ray form would
 // keep a few CUs busy while the rest of the GPU idles.
 template <int MODE, int KMAX, int SMAX, int LAY, bool PR, int NW>
 __global__ __launch_bounds__(kBlock) void sample_list_wave_kernel(SampleOpts o, SampleOut out, ViewArgs view,
@@ -91,7 +91,8 @@ __global__ __launch_bounds__(kBlock) void sample_list_wave_kernel(SampleOpts o, 
 template <int MODE, int KMAX, int SMAX, int LAY, bool PR, int NW>
 void launch_kernels(const SampleOpts& o, const SampleOut& out, const ViewArgs& view, const int* rays, int64_t R,
                 const TilePlan& tp, hipStream_t st) {
-    if (rays && R <= o.list_wave) {
+    // run_ray_wave holds the window's lanes in NW words; wider windows (k > 16) have more
+    if (rays && R <= o.list_wave && o.L <= 64 * NW) {
         sample_list_wave_kernel<MODE, KMAX, SMAX, LAY, PR, NW>
             <<<dim3((unsigned)ceil_div(R, kBlock / kWave)), dim3(kBlock), 0, st>>>(o, out, view, rays, R);
     } else if (rays) {
