@@ -445,8 +445,9 @@ def bench_per_view(args, wl):
             npts.knn_sampling(cs, opt, idx, table, radius=radius, mode=args.mode, feat=feat, s_max=s_max)
 
         t0 = time.perf_counter()
-        best, _ = autotune.tune(f"view/{wl['name']}/{args.mode}", one, reps=2, heavy=(C.HEAVY_DEFAULT, 512, 2048, 0),
-                                log=log)
+        form = C.sampling_form(opt, n, cs.height, cs.width, live=s_max)
+        best, _ = autotune.tune(f"view/{wl['name']}/{args.mode}/form{form}", one, reps=2, log=log,
+                                **autotune.knobs(form, heavy=(C.HEAVY_DEFAULT, 512, 2048, 0)))
         log(f"autotune: best {best} in {time.perf_counter() - t0:.1f} s")
         del idx, depth, table
     autotune.apply(best)

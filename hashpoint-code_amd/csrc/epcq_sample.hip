@@ -358,9 +358,8 @@ constexpr int64_t kRowsSparse = 10;
 // (with per-point radii the caller's s_max stands for that bound; a ray that
 // visits more is run by a whole wave), and a workspace for the point copy and
 // the queue of deferred rays.
-int takes_rows(SampleOpts& o, const epcq_camera* cam, int64_t n, int live_bound, bool compact,
-               const void* workspace, size_t workspace_bytes) {
-    const int64_t P = (int64_t)cam->width * cam->height;
+int takes_rows(SampleOpts& o, int64_t P, int64_t n, int live_bound, bool compact, const void* workspace,
+               size_t workspace_bytes) {
     if (o.k > kRowMaxK || live_bound > 2 || !workspace || workspace_bytes < sampling_bytes(n, P)) return kRowsNone;
     const int64_t d = (int64_t)o.L * n / std::max<int64_t>(P, 1);
     // candidates that the launch gives a lane of each SIMD: a ray with far more
@@ -556,6 +555,16 @@ extern "C" size_t epcq_sampling_workspace_size(int64_t n, int32_t height, int32_
     return sampling_bytes(n, (int64_t)height * width);
 }
 
+extern "C" int32_t epcq_sampling_form(const epcq_options* opt, int64_t n, int32_t height, int32_t width, int32_t live,
+                                      int32_t compact, int64_t rays, size_t workspace_bytes) {
+    static_assert(kRowsNone == EPCQ_FORM_LANE_SETS && kRowsTiles == EPCQ_FORM_ROW_TILES && kRowsWave == EPCQ_FORM_ROW_WAVES,
+                  "the forms' numbers");
+    if (!opt || height <= 0 || width <= 0 || n < 0) return EPCQ_FORM_LANE_SETS;
+    SampleOpts o = make_opts(nullptr, opt, nullptr);
+    if (rays >= 0) return takes_rows_list(o, rays, live);
+    return takes_rows(o, (int64_t)height * width, n, live, compact != 0, &o, workspace_bytes);
+}
+
 extern "C" int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camera* cam, const epcq_options* opt,
                                    const int32_t* sorted_idx, const int32_t* hash, int32_t mode, float* sp_xyz,
                                    int32_t* pc_idx, float* sp_t, uint8_t* mask, void* workspace,
@@ -570,7 +579,7 @@ extern "C" int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camer
     if (opt->num_sample_points_per_ray == 0) return EPCQ_OK;
     const int bound = epcq_max_live_samples(opt, opt->radius_threshold);
     SampleOpts o = make_opts(xyz, opt, nullptr);
-    o.rows = takes_rows(o, cam, n, bound, false, workspace, workspace_bytes);
+    o.rows = takes_rows(o, (int64_t)cam->width * cam->height, n, bound, false, workspace, workspace_bytes);
     SampleOut out{};
     out.sp_xyz = sp_xyz;
     out.pc_idx = pc_idx;
@@ -644,7 +653,7 @@ extern "C" int epcq_knn_sampling(const float* xyz, int64_t n, const epcq_camera*
     out.agg = agg;
     const int64_t nr = rays ? R : (int64_t)cam->width * cam->height;
     const int live = radius ? s_max : epcq_max_live_samples(opt, opt->radius_threshold);
-    o.rows = rays ? takes_rows_list(o, nr, live) : takes_rows(o, cam, n, live, true, workspace, workspace_bytes);
+    o.rows = rays ? takes_rows_list(o, nr, live) : takes_rows(o, nr, n, live, true, workspace, workspace_bytes);
     hipStream_t st = as_stream(stream);
     ViewArgs view = make_view(cam, sorted_idx, hash);
     prepare_bounds(o, view, n, cam, sorted_idx, hash, workspace, workspace_bytes, rays ? R : -1, st);

@@ -4,7 +4,8 @@ The full-image samplers take a tile shape (tile_w x tile_h rays per block),
 a staging capacity (points of a tile's halo region copied to LDS), a flag
 (XCD-contiguous tile order) and the outlier threshold of the wave-wide form
 (`heavy`); the best choice
-depends on the point density per pixel and the image sizes.  tune() times a
+depends on the point density per pixel and the image sizes.  A call over the
+rows of the point list reads few of these or none (knobs()).  tune() times a
 caller-supplied workload under candidate settings with HIP events and keeps
 the fastest, searching one knob at a time (shape, then capacity, then flags, then heavy).
 Results are cached per (device, key) in memory and, when EPCQ_TUNE_CACHE
@@ -106,6 +107,16 @@ def tune(key, run, reps=3, stream=None, shapes=SHAPES, caps=CAPS, flags=FLAGS, h
     _cache[full_key] = {"best": best, "times": times}
     _store()
     return dict(best), times
+
+
+def knobs(form, heavy=HEAVY):
+    """The settings that tune() has to try for a call of this form
+    (csrc.sampling_form): a knob that the form does not read keeps its default,
+    which other calls of the process then take too."""
+    if form == _C.FORM_LANE_SETS:
+        return {"heavy": tuple(heavy)}
+    fixed = {"shapes": (), "caps": (), "flags": ()}
+    return dict(fixed, heavy=tuple(heavy) if form == _C.FORM_ROW_TILES else ())
 
 
 def apply(tuning):

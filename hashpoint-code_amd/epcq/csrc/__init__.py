@@ -63,6 +63,9 @@ class _Tuning(ctypes.Structure):
 
 TUNE_XCD_ORDER = 1
 
+# epcq_sampling_form
+FORM_LANE_SETS, FORM_ROW_TILES, FORM_ROW_WAVES = 0, 1, 2
+
 
 class _ViewDesc(ctypes.Structure):
     _fields_ = [("xyz", ctypes.c_void_p), ("n", ctypes.c_int64), ("c2w", ctypes.c_float * 12),
@@ -109,6 +112,7 @@ ABI_SYMBOLS = {
     "epcq_quick_sampling_rays": (_I32, [_P, _I64, ctypes.POINTER(_Camera), ctypes.POINTER(_Options), _P, _P,
                                         _I32, _P, _I64, _P, _P, _P, _P, _P, _SZ, _P]),
     "epcq_sampling_workspace_size": (_SZ, [_I64, _I32, _I32]),
+    "epcq_sampling_form": (_I32, [ctypes.POINTER(_Options), _I64, _I32, _I32, _I32, _I32, _I64, _SZ]),
     "epcq_quick_query": (_I32, [_P, _I64, ctypes.POINTER(_Camera), ctypes.POINTER(_Options), _P, _P, _P,
                                 _I64, _P, _P]),
     "epcq_knn_sampling": (_I32, [_P, _I64, ctypes.POINTER(_Camera), ctypes.POINTER(_Options), _P, _P, _P,
@@ -413,6 +417,20 @@ def _workspace(n, H, W, device, cull):
     return torch.empty(int(_lib.epcq_sampling_workspace_size(n, H, W)), dtype=torch.uint8, device=device)
 
 
+def sampling_form(options, n, height, width, live=None, compact=True, rays=-1, workspace_bytes=None):
+    """FORM_* of a sampler call on n points and a height x width image: live
+    samples per ray (default: of the options and their radius), the compact or
+    the dense layout, the length of the ray list (-1: the image), and the
+    workspace (default: what the samplers allocate)."""
+    opts = _options_struct(options)
+    if live is None:
+        live = _lib.epcq_max_live_samples(ctypes.byref(opts), float(options.radius_threshold))
+    if workspace_bytes is None:
+        workspace_bytes = _lib.epcq_sampling_workspace_size(n, height, width)
+    return int(_lib.epcq_sampling_form(ctypes.byref(opts), n, height, width, int(live), int(compact), int(rays),
+                                       workspace_bytes))
+
+
 def _nbytes(t):
     return 0 if t is None else t.numel() * t.element_size()
 
@@ -494,7 +512,9 @@ def set_tuning(tile_w=32, tile_h=8, tile_cap=1024, flags=0, heavy=HEAVY_DEFAULT,
     block, tile_cap points staged in LDS per tile, TUNE_* flags; rays whose
     unculled window buckets hold more than `heavy` points are sampled by a
     whole wave (0: never); ray lists of at most `list_wave` rays are sampled
-    one wave per ray (0: never)."""
+    one wave per ray (0: never).  Which fields a call reads depends on its
+    form (sampling_form): the lane sets read all, the tiles over rows `heavy`
+    alone, and one wave per ray none."""
     _raise_on(_lib.epcq_set_tuning(ctypes.byref(_Tuning(int(tile_w), int(tile_h), int(tile_cap), int(flags),
                                                         int(heavy), int(list_wave)))))
 

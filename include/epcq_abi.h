@@ -79,10 +79,12 @@ const char* epcq_last_error(void);
  * wave (64 lanes share its candidate walks) after the tile's other rays,
  * instead of by one lane; 0 never does.  list_wave: a ray list (the rays
  * argument of the samplers) of at most this many rays is sampled one wave per
- * ray, longer ones one lane per ray; 0 never does.  The row-run sampler, which
- * takes most full images given a workspace, has tiles of its own and reads
- * heavy as 8 to 32 times that many points.  Results are identical either way.
- * Process-wide, guarded by a mutex; the autotuner sets it.
+ * ray, longer ones one lane per ray; 0 never does.  Which fields a call reads
+ * depends on its form (epcq_sampling_form): EPCQ_FORM_LANE_SETS reads all but
+ * list_wave, EPCQ_FORM_ROW_TILES has tiles of its own and reads heavy as 8 to
+ * 32 times that many points, EPCQ_FORM_ROW_WAVES reads none; ray lists read
+ * list_wave, and heavy where they are lane sets.  Results are identical either
+ * way.  Process-wide, guarded by a mutex; the autotuner sets it.
  * Defaults: 32, 8, 1024, 0, 128, 65536.
  */
 typedef struct epcq_tuning {
@@ -199,6 +201,17 @@ int epcq_quick_sampling_rays(const float* xyz, int64_t n, const epcq_camera* cam
  * smaller workspace the samplers skip nothing and gather the points through
  * sorted_idx (same results). */
 size_t epcq_sampling_workspace_size(int64_t n, int32_t height, int32_t width);
+
+/*
+ * The form a sampler call takes (a host helper without state of its own): the
+ * lane-set kernels, tiles over the rows of the point list, or one wave per ray
+ * over these.  live: epcq_max_live_samples of the options (with per-point
+ * radii, the call's s_max); compact: epcq_knn_sampling's layout, else the dense
+ * one; rays: length of the ray list, or -1 for the image.
+ */
+enum epcq_sampling_forms { EPCQ_FORM_LANE_SETS = 0, EPCQ_FORM_ROW_TILES = 1, EPCQ_FORM_ROW_WAVES = 2 };
+int32_t epcq_sampling_form(const epcq_options* opt, int64_t n, int32_t height, int32_t width, int32_t live,
+                           int32_t compact, int64_t rays, size_t workspace_bytes);
 
 /*
  * quick_query_for_nearby_point -- replaces `quick_query_for_nearby_point`

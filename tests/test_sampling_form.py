@@ -1,0 +1,47 @@
+"""Which form a sampler call takes, and that the autotuner varies only what the
+form reads (host only)."""
+import epcq.csrc as C
+from epcq import autotune
+from epcq.epcq import RenderOptions
+
+
+def form(n, W, H, rays=-1, live=None, compact=True, ws=None, **opt):
+    return C.sampling_form(RenderOptions(**opt), n, H, W, live=live, compact=compact, rays=rays, workspace_bytes=ws)
+
+
+def test_forms():
+    assert form(1_000_000, 800, 800) == C.FORM_ROW_TILES
+    assert form(1_000_000, 800, 800, compact=False) == C.FORM_ROW_TILES
+    assert form(1_000_000, 200, 150) == C.FORM_ROW_WAVES
+    # not over rows: no workspace, one of the former size, wide windows, more live samples
+    full = C._lib.epcq_sampling_workspace_size(1_000_000, 800, 800)
+    for kw in (dict(ws=0), dict(ws=full - 1), dict(kernel_size=17), dict(live=3),
+               dict(sdf2weight_gaussian_gamma=0.2, sdf2weight_gaussian_alpha=0.01)):
+        assert form(1_000_000, 800, 800, **kw) == C.FORM_LANE_SETS, kw
+    # lists by their length
+    old = C.get_tuning()
+    try:
+        C.set_tuning(**dict(old, list_wave=100))
+        assert form(1_000_000, 800, 800, rays=100, ws=0) == C.FORM_ROW_WAVES
+        assert form(1_000_000, 800, 800, rays=101) == C.FORM_LANE_SETS
+    finally:
+        C.set_tuning(**old)
+
+
+def test_autotuner_varies_what_the_form_reads(monkeypatch):
+    monkeypatch.setattr(autotune.torch.cuda, "get_device_name", lambda: "none")
+    monkeypatch.setattr(autotune, "time_ms", lambda fn, **kw: fn())
+    monkeypatch.setattr(autotune, "_cache", {"": 0})
+    seen = []
+
+    def run(t):  # every other setting is faster than the default
+        seen.append(t)
+        return 2.0 if t == autotune.DEFAULT else 1.0 + 0.01 * len(seen)
+
+    best, _ = autotune.tune("waves", run, **autotune.knobs(C.FORM_ROW_WAVES))
+    assert best == autotune.DEFAULT and not seen
+    best, _ = autotune.tune("tiles", run, **autotune.knobs(C.FORM_ROW_TILES, heavy=(128, 512, 0)))
+    assert {k: v for k, v in best.items() if k != "heavy"} == {k: v for k, v in autotune.DEFAULT.items() if k != "heavy"}
+    assert sorted({t["heavy"] for t in seen}) == [0, 128, 512]
+    best, _ = autotune.tune("lanes", run, **autotune.knobs(C.FORM_LANE_SETS))
+    assert {(t["tile_w"], t["tile_h"]) for t in seen} >= set(autotune.SHAPES)
