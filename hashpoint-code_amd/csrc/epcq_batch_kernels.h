@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void batch_sample_kernel(BatchHeader* __restri
         // a tile whose halo region exceeds the LDS reads global memory right
         // away: the densest views come first, so these long tiles overlap
         // with the rest of the batch
-        const bool staged = sample_tile_body<MODE, KMAX, SMAX, kLayCompact, PR>(o, out, bv.view, tp,
+        const bool staged = sample_tile_body<MODE, KMAX, SMAX, kLayCompact, PR, 1, true>(o, out, bv.view, tp,
                                                                                 item - pf[v], bv.tiles_x,
                                                                                 bv.ray_off, sm);
         if (!staged)
