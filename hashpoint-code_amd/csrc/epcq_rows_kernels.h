@@ -55,9 +55,15 @@ __global__ __launch_bounds__(kRowWaveWaves* kWave) void sample_deferred_kernel(S
     run_queue<MODE, KMAX, LAY, PR>(o, out, view, row_queue(view)->count, sm[threadIdx.x / kWave]);
 }
 
+// Waves per SIMD of the form of one wave per ray: LDS holds four blocks per CU,
+// and the registers have to as well.  The feature layout takes what it needs (94
+// to 104 registers with buffers of 8, up to 213 with 32).
+template <int LAY>
+constexpr int kListWavesPerSimd = LAY != kLayFeat ? 4 : 1;
+
 // One wave per ray of a list, or of the whole image (rays null: R pixels).
 template <int MODE, int KMAX, int LAY, bool PR>
-__global__ __launch_bounds__(kRowWaveWaves* kWave) void sample_list_rows_kernel(SampleOpts o, SampleOut out,
+__global__ __launch_bounds__(kRowWaveWaves* kWave, kListWavesPerSimd<LAY>) void sample_list_rows_kernel(SampleOpts o, SampleOut out,
                                                                                 ViewArgs view,
                                                                                 const int* __restrict__ rays,
                                                                                 int64_t R) {

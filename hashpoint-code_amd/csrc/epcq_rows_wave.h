@@ -13,12 +13,14 @@
 // LDS; the walks then take these.  Where they are too many, the pass is
 // repeated without what lies more than kWaveDepth slots behind the first hit
 // found so far (a walk that would have to go on there starts again with every
-// candidate).  Where the table's buckets are not in row-major list order, every
+// candidate).  Where that leaves too many as well, what is listed is the chunks
+// of 64 that hold a candidate within the bound, and the walks take all of
+// these.  Where the table's buckets are not in row-major list order, every
 // bucket is a segment of its own.
 //
 // The 48-hit cap counts hits per bucket: where a bucket holds more points than
 // that, each candidate's bucket is found from its row's column starts, and the
-// depth limit is off.
+// depth limit is off; a walk over the hits leaves a bucket after its 48th.
 //
 // The order-dependent steps are those of run_ray_wave: sums and neighbours
 // take the candidates in the canonical order, lowest lane first.
@@ -26,7 +28,12 @@
 // What bounds it: the latency of those two waits on a short list (4096 rays of
 // 1M points at 800 x 800, k = 5: 57 -> 32 us against run_ray_wave), instruction
 // issue on an image (600k points at 160 x 100, k = 9, build included: 1.82 ->
-// 0.22 ms against the lane-set tiles).
+// 0.22 ms against the lane-set tiles), and the densest ray's wave where most of
+// the points fall to few pixels.  The chunk list and the end at the 48th hit are
+// for those, against walks over all candidates: 2726 rays of 1.4M points at 224
+// x 170, k = 5, 1.41 -> 0.56 ms (lane sets 0.84); an image of 1.3M points at 240
+// x 136, k = 15, 3.90 -> 1.07; over 150 images without features 2.6 % on
+// average, over 500 lists 0.8 %, and neither way for most.
 #pragma once
 
 #include "epcq_rows.h"
@@ -43,9 +50,15 @@ struct RowWaveSmem {
     uint8_t row[kRowMaxK * kRowMaxK];  // its window row, or kOneBucket
     int col[kRowMaxK][kRowMaxK];       // per window row and column: where the first bucket at or right of it starts
     int hist[kMaxSlots];               // hits per depth slot
-    int pos[kWaveList];                // list positions that pass the bound
+    int pos[kWaveList];                // list positions that pass the bound, or first ones of chunks
     uint8_t seg[kWaveList];            // their segments
 };
+
+// What the walks of a ray go over: the segments' candidates, or the positions in
+// pos; for a ray of more than these hold (its own instance of the walks, so that
+// the others stay short), the chunks that start at the positions in pos, or all
+// candidates where they are too many as well.
+enum RowWaveOver { kOverAll, kOverList, kOverChunks };
 
 // List point j and the squared threshold of its radius, from the pixel-ordered
 // copies where there are any.
@@ -114,13 +127,13 @@ __device__ __forceinline__ void row_wave_write(const SampleOpts& o, const Sample
     }
 }
 
-// The walks of one ray over its N candidates (the listed positions, or all C
-// of the segments) and its outputs.  Returns true when the list left out
-// (`dropped`) what the walk needs; nothing written then stays.
-template <int MODE, int KMAX, int LAY, bool PR>
+// The walks of one ray over its N candidates (all C of the segments, the listed
+// positions, or 64 for each listed chunk) and its outputs.  Returns true when
+// the list left out (`dropped`) what the walk needs; nothing written then stays.
+template <int MODE, int KMAX, int LAY, bool PR, bool MANY>
 __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const SampleOut& out, const RowList<PR>& src,
                                                const Ray& ray, int64_t ri, RowWaveSmem& sm, int nseg, int64_t C,
-                                               int64_t N, bool listed, bool dropped, bool capped) {
+                                               int64_t N, RowWaveOver over, bool dropped, bool capped) {
     const int lane = __lane_id();
     // ---- candidates, 64 at a time
     struct Cand {
@@ -132,6 +145,10 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
     struct Carry {
         int seg, kept;
     };
+    auto segment_end = [&](int seg) {  // the list position after it
+        const int64_t p1 = seg + 1 < nseg ? sm.pre[seg + 1] : C;
+        return (sm.st[seg] & 0x7fffffff) + (int)(p1 - sm.pre[seg]);
+    };
     auto load = [&](int64_t c0) {
         Cand x;
         const int64_t i = c0 + lane;
@@ -140,11 +157,16 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
         x.dup = false;
         x.p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         x.lim = 0.0f;
+        if (MANY && over == kOverChunks)
+            x.in = x.in && sm.pos[c0 / kWave] + lane < segment_end(sm.seg[c0 / kWave]);
         if (x.in) {
             int j;
-            if (listed) {
+            if (!MANY && over == kOverList) {
                 x.seg = sm.seg[i];
                 j = sm.pos[i];
+            } else if (MANY && over == kOverChunks) {
+                x.seg = sm.seg[c0 / kWave];
+                j = sm.pos[c0 / kWave] + lane;
             } else {
                 int lo = 0, hi = nseg;  // last segment that starts at or before i
                 while (hi - lo > 1) {
@@ -185,29 +207,46 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
             const uint64_t own = hb & (~0ull << from) & (next ? (1ull << (__ffsll((unsigned long long)next) - 1)) - 1ull
                                                               : ~0ull);
             x.keep = hit && __popcll(own & lanemask_lt()) + (x.seg == cy.seg ? cy.kept : 0) < kSampleLaneHits;
-            const int last = (int)min<int64_t>(kWave, N - c0) - 1;
+            const int last = MANY ? 63 - __clzll((long long)__ballot(x.in))  // the lanes of a chunk come first
+                                  : (int)min<int64_t>(kWave, N - c0) - 1;
             const int total = __popcll(own) + (x.seg == cy.seg ? cy.kept : 0);
             cy.kept = lane_bcast(total, last);
             cy.seg = lane_bcast(x.seg, last);
         }
     };
-    Cand cache[kWaveCache];
+    constexpr int kCache = MANY ? 0 : kWaveCache;  // chunks kept for all walks
+    Cand cache[MANY ? 1 : kWaveCache];
 #pragma unroll
-    for (int q = 0; q < kWaveCache; ++q) cache[q] = load((int64_t)q * kWave);
+    for (int q = 0; q < kCache; ++q) cache[q] = load((int64_t)q * kWave);
     Carry cy0{-1, 0};
 #pragma unroll
-    for (int q = 0; q < kWaveCache; ++q)
+    for (int q = 0; q < kCache; ++q)
         if ((int64_t)q * kWave < N) test(cache[q], (int64_t)q * kWave, cy0);
         else cache[q].keep = false;
-    auto walk = [&](auto&& fn) {
+    // The next chunk of a walk over the hits: where the bucket visit that the
+    // last one ended in has given its 48, not before the visit's end (a bucket
+    // may hold tens of thousands of points).
+    auto past_full = [&](int64_t c0, const Carry& cy) -> int64_t {
+        if (!MANY || !capped || cy.kept < kSampleLaneHits) return c0;
+        const int seg = cy.seg / kRowMaxK, col = cy.seg % kRowMaxK, r = sm.row[seg];
+        const int st = sm.st[seg] & 0x7fffffff;
+        const int end = r != kOneBucket && col + 1 < o.k ? sm.col[r][col + 1] : segment_end(seg);
+        if (over == kOverAll) return max<int64_t>(c0, sm.pre[seg] + (end - st));
+        while (c0 < N && sm.seg[c0 / kWave] == seg && sm.pos[c0 / kWave] + kWave <= end) c0 += kWave;
+        return c0;
+    };
+    auto walk = [&](bool hits, auto&& fn) {
 #pragma unroll
-        for (int q = 0; q < kWaveCache; ++q)
+        for (int q = 0; q < kCache; ++q)
             if ((int64_t)q * kWave < N) fn(cache[q]);
         Carry cy = cy0;
-        for (int64_t c0 = (int64_t)kWaveCache * kWave; c0 < N; c0 += kWave) {
+        int64_t c0 = (int64_t)kCache * kWave;
+        while (c0 < N) {
             Cand x = load(c0);
             test(x, c0, cy);
             fn(x);
+            c0 += kWave;
+            if (hits) c0 = past_full(c0, cy);
         }
     };
 
@@ -215,7 +254,7 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
     int ns = 0;
     float ts_arr[2] = {0.0f, 0.0f};
     float tmin = 1e3f, tmax = -1e3f;
-    walk([&](const Cand& x) {
+    walk(true, [&](const Cand& x) {
         if (x.keep) {
             tmin = tmin > x.t ? x.t : tmin;
             tmax = tmax < x.t ? x.t : tmax;
@@ -229,7 +268,7 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
             const float qf = (x.t - tmin) / o.t_intvl;
             return x.keep && qf > -1.0f && qf < (float)kMaxSlots ? (int)qf : -1;
         };
-        walk([&](const Cand& x) {
+        walk(true, [&](const Cand& x) {
             const int s = slot(x);
             if (s >= 0) atomicAdd(&sm.hist[s], 1);
         });
@@ -255,7 +294,7 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
                 b &= b - 1ull;
                 const int sl = half * kWave + x;
                 float sum = 0.0f;
-                walk([&](const Cand& h) {
+                walk(true, [&](const Cand& h) {
                     const bool in_slot = slot(h) == sl;
                     const float dist = in_slot ? sqrtf(h.e2) : 0.0f;
                     for (uint64_t m = __ballot(in_slot); m; m &= m - 1ull)
@@ -288,7 +327,7 @@ __device__ __forceinline__ bool row_wave_walks(const SampleOpts& o, const Sample
         const float s0 = ray.o[0] + ts * ray.d[0], s1 = ray.o[1] + ts * ray.d[1], s2 = ray.o[2] + ts * ray.d[2];
         NbBuf<MODE, KMAX> buf;
         buf.init();
-        walk([&](const Cand& x) {
+        walk(false, [&](const Cand& x) {
             const float d2 = sqnorm3(s0 - x.p.x, s1 - x.p.y, s2 - x.p.z);
             const bool take = x.in && within(d2, x.lim) && !(MODE == EPCQ_MODE_KNN && x.dup);
             const float d = take ? sqrtf(d2) : 0.0f;
@@ -386,12 +425,33 @@ __device__ __forceinline__ void run_ray_rows(const SampleOpts& o, const SampleOu
     wave_lds_fence();
 
     // ---- the positions that pass the bound, four chunks in flight
-    bool listed = C > kWaveCache * kWave;
     bool dropped = false;  // something beyond the list's depth was left out
     int64_t N = C;         // candidates of the walks
-    if (listed) {
-        const RowFrame f = row_frame(view.c2w);
+    RowWaveOver over = kOverAll;
+    // the bounds of 4 chunks of segment positions [st + c0, st + len)
+    auto bounds = [&](const RowFrame& f, const RowRay& rr, int st, int len, int c0, float4 (&cd)[4], bool (&pass)[4]) {
         const float r0 = __builtin_amdgcn_sqrtf(o.r2lim);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = c0 + q * kWave + lane;
+            if (i >= len) continue;
+            if (view.cand) {
+                cd[q] = view.cand[st + i];
+            } else {
+                const float4 p = src.point(st + i);
+                cd[q] = row_candidate(f, p, PR ? __builtin_amdgcn_sqrtf(src.limit(o, st + i, p)) : r0);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float da = cd[q].x - rr.a, db = cd[q].y - rr.b;
+            pass[q] = c0 + q * kWave + lane < len && !(__builtin_fmaf(db, db, da * da) > cd[q].z * rr.g);
+        }
+    };
+    auto segment_length = [&](int s) { return uniform((int)((s + 1 < nseg ? sm.pre[s + 1] : C) - sm.pre[s])); };
+    bool many = false;  // too many for the list
+    if (C > kWaveCache * kWave) {
+        const RowFrame f = row_frame(view.c2w);
         const RowRay rr = row_ray(view.c2w, ray);
         const float depth = (float)(kWaveDepth + 1) * o.t_intvl;
         const float inf = __builtin_inff();
@@ -399,28 +459,11 @@ __device__ __forceinline__ void run_ray_rows(const SampleOpts& o, const SampleOu
         int n = 0;
         bool cut = false;
         for (int s = 0; s < nseg; ++s) {
-            const int st = uniform(sm.st[s]) & 0x7fffffff;
-            const int64_t p0 = sm.pre[s], p1 = s + 1 < nseg ? sm.pre[s + 1] : C;
-            const int len = uniform((int)(p1 - p0));
+            const int st = uniform(sm.st[s]) & 0x7fffffff, len = segment_length(s);
             for (int c0 = 0; c0 < len; c0 += 4 * kWave) {
                 float4 cd[4];
                 bool pass[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int i = c0 + q * kWave + lane;
-                    if (i >= len) continue;
-                    if (view.cand) {
-                        cd[q] = view.cand[st + i];
-                    } else {
-                        const float4 p = src.point(st + i);
-                        cd[q] = row_candidate(f, p, PR ? __builtin_amdgcn_sqrtf(src.limit(o, st + i, p)) : r0);
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float da = cd[q].x - rr.a, db = cd[q].y - rr.b;
-                    pass[q] = c0 + q * kWave + lane < len && !(__builtin_fmaf(db, db, da * da) > cd[q].z * rr.g);
-                }
+                bounds(f, rr, st, len, c0, cd, pass);
                 if (cut) {
                     // hits ahead of the front move it (first where none is known)
 #pragma unroll
@@ -459,18 +502,57 @@ __device__ __forceinline__ void run_ray_rows(const SampleOpts& o, const SampleOu
                 s = -1;
             }
         }
-        listed = n <= kWaveList;
-        if (listed) N = n;
-        else dropped = false;
+        many = n > kWaveList;
+        if (!many) {
+            over = kOverList;
+            N = n;
+        }
         wave_lds_fence();
     }
-    while (row_wave_walks<MODE, KMAX, LAY, PR>(o, out, src, ray, ri, sm, nseg, C, N, listed, dropped, capped)) {
-        // the walk has to go on beyond the list's depth: with every candidate
-        listed = dropped = false;
-        N = C;
-        sm.hist[lane] = 0;
-        sm.hist[lane + kWave] = 0;
+    // (in the feature layout a ray of too many walks all of its candidates: a
+    // second instance of the sums cost all rays 2 % there, in scalar spills)
+    constexpr bool kChunks = LAY != kLayFeat;
+    if (!many || !kChunks) {
+        dropped = dropped && !many;
+        while (row_wave_walks<MODE, KMAX, LAY, PR, false>(o, out, src, ray, ri, sm, nseg, C, N, over, dropped, capped)) {
+            // the walk has to go on beyond the list's depth
+            many = true;
+            dropped = false;
+            over = kOverAll;
+            N = C;
+            sm.hist[lane] = 0;
+            sm.hist[lane + kWave] = 0;
+            wave_lds_fence();
+            if (kChunks) break;
+        }
+        if (!many || !kChunks) return;
+    }
+    if constexpr (kChunks) {
+        // ---- the chunks that hold a position within the bound, at any depth
+        const RowFrame f = row_frame(view.c2w);
+        const RowRay rr = row_ray(view.c2w, ray);
+        int n = 0;
+        for (int s = 0; s < nseg && n <= kWaveList; ++s) {
+            const int st = uniform(sm.st[s]) & 0x7fffffff, len = segment_length(s);
+            for (int c0 = 0; c0 < len && n <= kWaveList; c0 += 4 * kWave) {
+                float4 cd[4];
+                bool pass[4];
+                bounds(f, rr, st, len, c0, cd, pass);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (!__any(pass[q])) continue;
+                    if (n < kWaveList && lane == 0) {
+                        sm.pos[n] = st + c0 + q * kWave;
+                        sm.seg[n] = (uint8_t)s;
+                    }
+                    ++n;
+                }
+            }
+        }
+        const bool chunks = n <= kWaveList;
         wave_lds_fence();
+        row_wave_walks<MODE, KMAX, LAY, PR, true>(o, out, src, ray, ri, sm, nseg, C, chunks ? (int64_t)n * kWave : C,
+                                                  chunks ? kOverChunks : kOverAll, false, capped);
     }
 }
 

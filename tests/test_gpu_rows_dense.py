@@ -113,6 +113,46 @@ def test_wave_lists_per_point_radius(dev):
     compact_vs_dense(v, "knn", rays=rng.integers(0, W * H, 600).astype(np.int32), feat=feat, cull=False)
 
 
+@pytest.mark.parametrize("hot,per_pixel,k,K,mode,opts", [
+    # buckets beyond the 48-hit cap, and more candidates within the bound than the list holds
+    (0, 70, 5, 8, "knn", dict()),
+    (0, 70, 9, 16, "knn", dict(num_sample_points_per_ray=1)),
+    (0, 70, 9, 8, "compat", dict(sdf2weight_gaussian_gamma=0.0005)),
+    (0, 130, 7, 32, "knn", dict(t_intvl=3e-4)),
+    # a bucket of more chunks than the list holds, beside ordinary ones
+    (90_000, 20, 5, 8, "knn", dict()),
+    (90_000, 20, 5, 8, "compat", dict()),
+    (90_000, 60, 9, 16, "knn", dict()),
+    # and one whose chunks it holds
+    (20_000, 20, 9, 8, "knn", dict()),
+    (20_000, 60, 3, 8, "compat", dict()),
+])
+def test_wave_full_buckets(dev, hot, per_pixel, k, K, mode, opts):
+    W, H = 44, 34
+    cam = camera(W, H)
+    rng = np.random.default_rng(hot + k)
+    pts = volume(cam, per_pixel, 3.0, 3.6, rng)
+    if hot:  # before one pixel, on two surfaces
+        z = rng.choice([3.0, 3.2], hot) + rng.normal(0, 0.01, hot)
+        pts = np.concatenate([pts, unproject(cam, 22 + rng.uniform(0.3, 0.7, hot), 17 + rng.uniform(0.3, 0.7, hot), z)])
+        pts = np.ascontiguousarray(pts[rng.permutation(len(pts))])
+    r = 0.2
+    v = View(pts, cam, dev, **dict(dict(kernel_size=k, radius_threshold=r, num_point_cloud_per_sp=K,
+                                        num_sample_points_per_ray=2), **opts))
+    assert C.sampling_form(v.opt, len(pts), H, W) == C.FORM_ROW_WAVES
+    most = v.oh[:, 1].max()
+    assert most > BUCKET and near_the_ray(v, 22, 17, r) > LIST
+    assert (most > 64 * LIST) == (hot == 90_000)
+    print("wave full buckets", hot, per_pixel, k, K, mode, flush=True)
+    check_dense(v, mode)
+    compact_vs_dense(v, mode)
+    rays = np.concatenate([rng.integers(0, W * H, 300), [17 * W + 22]]).astype(np.int32)
+    feat = torch.randn(len(pts), 9, generator=torch.Generator().manual_seed(3)).to(dev)
+    compact_vs_dense(v, mode, rays=rays)
+    compact_vs_dense(v, mode, rays=rays, cull=False)
+    compact_vs_dense(v, mode, rays=rays, feat=feat)
+
+
 def patched(cam, n, per_pixel, x0, y0, w, h, rng):
     """n points over the whole image and per_pixel before each pixel of a patch."""
     u, y = np.meshgrid(np.arange(x0, x0 + w), np.arange(y0, y0 + h))
