@@ -321,37 +321,58 @@ int takes_rows_list(const SampleOpts& o, int64_t R, int live_bound) {
     return o.k <= kRowMaxK && live_bound <= 2 && R <= o.list_wave ? kRowsWave : kRowsNone;
 }
 
-// Which form an image takes, by its pixels P and the points d that a ray's
-// window holds on average (measured with the build; tile form / wave form /
-// lane sets in ms):
-// - P <= kWaveImage: 64 rays per wave would leave SIMDs idle; waves.  1M points
-//   at 400 x 300, k = 5: 0.60 / 0.35 / 1.18; at 640 x 512: 0.47 / 0.69 / 1.1.
+// Which form an image takes, by its pixels P, its points n and the points d that
+// a ray's window holds on average.  The lines lie where the medians of 1,900
+// images (cameras, scenes, radii and buffers varied; call with the build, which
+// all forms share) cross: 0.68 of the lane sets' time in the geometric mean.  A
+// twentieth of the images are more than 3 % slower than these, single ones up to
+// 1.6 times, since how the points cluster is not known here.  Tile form / wave form /
+// lane sets in ms:
+// - P <= kWaveTiny: 64 rays per wave would leave SIMDs idle; waves.  260 x 147,
+//   k = 5, d = 156: 0.46 / 0.17 / 0.66; 203 x 152, k = 11, d = 202: 0.36 / 0.19 /
+//   0.29.
+// - windows of up to eight columns, P <= kWaveImage: waves from kWaveFew points
+//   on, below these the tiles, whose cost is the candidates rather than the rays:
+//   400 x 300, d = 2: 0.09 / 0.18 / 0.09 in a box, 0.10 / 0.18 / 0.13 on a sphere,
+//   d = 52: 0.51 / 0.27 / 0.67.  Rows of more than kWaveBuffer neighbours, whose
+//   buffers take the wave form 213 registers, from kWaveMid on: 386 x 292, k = 7,
+//   K = 32, d = 59: 0.34 / 0.92 / 0.47.
 // - up to four times as many: each tile is a long serial walk, and the longest
 //   ones end last.  Waves from kWaveDense points on (half the pixels: from
 //   kWaveMid): a sphere at 500 x 503, k = 7: d = 195 1.15 / 0.71 / 1.03, d =
 //   292 1.53 / 0.81 / 1.47; a box at 640 x 480, k = 7: d = 160 0.64 / 0.97 /
-//   0.92, d = 319 1.15 / 1.26 / 1.62; d = 4400 10.6 / 6.2 / 8.0.
-// - windows of more than eight columns, two blocks of whose tiles fit on a CU,
-//   cost more in both forms, and up to four times as many pixels (from 13
-//   columns on eight times) the lane sets are ahead from kWaveMid to kWaveWide
-//   points: k = 9 at 500 x 503, d = 298
-//   0.86 / 1.04 / 0.89 in a box and 1.92 / 0.88 / 1.02 on a sphere; k = 11 at
-//   640 x 480, d = 364 1.34 / 1.40 / 1.19; k = 15 at 800 x 800, d = 351 1.67 /
-//   - / 1.52; but k = 9 at 800 x 800, d = 253 2.27 / - / 2.82, at 500 x 503, d =
-//   484 3.59 / 1.01 / 1.53, and k = 15 at 1920 x 1080, d = 217 2.66 / - / 5.56.
+//   0.92, d = 319 1.15 / 1.26 / 1.62; d = 4400 10.6 / 6.2 / 8.0.  Not with more than
+//   kWaveBuffer neighbours: 621 x 350, k = 7, K = 32, d = 138: waves 2.7, lane sets
+//   1.7, and tiles 0.7 of these in the median.
+// - wider windows, two blocks of whose tiles fit on a CU, cost more in both
+//   forms.  Waves from kWaveFull points per pixel on, up to twice kWaveImage (345
+//   x 261, k = 9, d = 3240: 3.8 / 1.0 / 4.6), and from kWaveFullest on up to four
+//   times (685 x 683, k = 9, d = 279: 1.13 / 1.63 / 1.00); of twice these with more
+//   than kWaveBuffer neighbours.  Below that the lane
+//   sets, up to twice kWaveImage (400 x 340, k = 9, d = 35: 0.25 / 0.33 / 0.19;
+//   500 x 503, k = 13, d = 90: 0.56 / 0.75 / 0.45), and from kWaveMid points on
+//   up to four times (k = 11 at 640 x 480, d = 364 1.34 / 1.40 / 1.19), from 13
+//   columns on eight times, there below kWaveWide (k = 15 at 800 x 800, d = 351
+//   1.67 / - / 1.52).  The other images take the tiles: medians of 0.76 of the lane
+//   sets' time at two to four times kWaveImage, 0.65 at four to eight, 0.4 above.
+constexpr int64_t kWaveTiny = 40000;
 constexpr int64_t kWaveImage = 131072;
+constexpr int64_t kWaveFew = 25;
 constexpr int64_t kWaveMid = 100;
 constexpr int64_t kWaveDense = 256;
 constexpr int64_t kWaveWide = 400;
+constexpr int64_t kWaveFull = 3, kWaveFullest = 5;
+constexpr int kWaveBuffer = 16;
 
-// Where a window holds fewer than ten points on average, a ray has next to
-// nothing to test, and the rows' bounds and the S * K slots of the dense
-// layout are what is left: there the lane sets stay ahead.  Measured, rows
-// against lane sets, 800 x 800 pixels, k = 5, dense layout: 0.19 against 0.16
-// ms with 100k points, 0.24 against 0.21 with 200k, 0.27 against 0.26 with
-// 300k, 0.33 against 0.39 with 600k; in the compact layout rows are ahead at
-// each of these (200k points at 1600 x 1200, k = 3: 0.31 against 0.36).
-constexpr int64_t kRowsSparse = 10;
+// Where a window holds few points on average, a ray has next to nothing to test,
+// and the rows' bounds and the fills are what is left: there the lane sets stay
+// ahead.  Fewer than ten in the dense layout; measured, rows against lane sets, 800
+// x 800 pixels, k = 5: 0.19 against 0.16 ms with 100k points, 0.24 against 0.21
+// with 200k, 0.27 against 0.26 with 300k, 0.33 against 0.39 with 600k.  Fewer than
+// five in the compact layout: 963 x 964, k = 5, d = 4: 0.38 against 0.32, 1635 x
+// 1636, k = 3, d = 1: 0.48 against 0.36; the medians of 110 images are even below
+// five and at 0.89 from there on.
+constexpr int64_t kRowsSparse = 10, kRowsSparseCompact = 5;
 
 // Whether a full image takes the row-run sampler (epcq_rows.h): windows that
 // its LDS rows hold, options under which a ray can visit two slots at most
@@ -365,14 +386,22 @@ int takes_rows(SampleOpts& o, int64_t P, int64_t n, int live_bound, bool compact
     // candidates that the launch gives a lane of each SIMD: a ray with far more
     // would outlast the others
     o.row_heavy = (int)std::min<int64_t>(kRowHeavyMost, std::max<int64_t>(kRowHeavyLeast, (int64_t)o.L * n / (65536 * 128)));
-    if (P <= kWaveImage) return kRowsWave;
-    if (!compact && d < kRowsSparse) return kRowsNone;
-    if (o.k > 8) {
-        if (P <= 4 * kWaveImage && d >= kWaveWide) return kRowsWave;
-        if (P <= (o.k > 12 ? 8 : 4) * kWaveImage && d >= kWaveMid && d < kWaveWide) return kRowsNone;
-        return kRowsTiles;
+    const bool wide = o.k > 8, large = o.Kc > kWaveBuffer;
+    if (P <= kWaveTiny) return kRowsWave;
+    if (wide) {
+        const int64_t full = (P <= 2 * kWaveImage ? kWaveFull : kWaveFullest) * (large ? 2 : 1);
+        if (P <= 4 * kWaveImage && n >= full * P) return kRowsWave;
+        if (P <= 2 * kWaveImage) return kRowsNone;
+    } else if (P <= kWaveImage && d >= (large ? kWaveMid : kWaveFew)) {
+        return kRowsWave;
     }
-    if (P <= 4 * kWaveImage && d >= (P <= 2 * kWaveImage ? kWaveMid : kWaveDense)) return kRowsWave;
+    if (d < (compact ? kRowsSparseCompact : kRowsSparse)) return kRowsNone;
+    if (wide) {
+        if (P <= 4 * kWaveImage) return d >= kWaveMid ? kRowsNone : kRowsTiles;
+        return o.k > 12 && P <= 8 * kWaveImage && d >= kWaveMid && d < kWaveWide ? kRowsNone : kRowsTiles;
+    }
+    if (!large && P > kWaveImage && P <= 4 * kWaveImage && d >= (P <= 2 * kWaveImage ? kWaveMid : kWaveDense))
+        return kRowsWave;
     return kRowsTiles;
 }
 

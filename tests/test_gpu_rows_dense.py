@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import epcq.csrc as C
+import test_gpu_rows
 from epcq import synth
 from epcq.epcq import RenderOptions
 from scenes import bits, to_dev
@@ -167,17 +168,17 @@ def patched(cam, n, per_pixel, x0, y0, w, h, rng):
 
 TILES = [
     # W, H, k, K, mode, points over the image, points per pixel and patch, features, per-point radius, S
-    (400, 330, 16, 16, "knn", 40_000, 0, (0, 0, 0, 0), 32, True),
-    (400, 330, 16, 16, "compat", 40_000, 0, (0, 0, 0, 0), 7, False),
-    (430, 310, 11, 9, "knn", 60_000, 0, (0, 0, 0, 0), 5, False),
-    (430, 310, 9, 16, "compat", 80_000, 0, (0, 0, 0, 0), 0, True),
-    (430, 310, 12, 12, "knn", 60_000, 0, (0, 0, 0, 0), 0, False),
+    (640, 420, 16, 16, "knn", 40_000, 0, (0, 0, 0, 0), 32, True),
+    (640, 420, 16, 16, "compat", 40_000, 0, (0, 0, 0, 0), 7, False),
+    (650, 410, 11, 9, "knn", 60_000, 0, (0, 0, 0, 0), 5, False),
+    (650, 410, 9, 16, "compat", 80_000, 0, (0, 0, 0, 0), 0, True),
+    (650, 410, 12, 12, "knn", 60_000, 0, (0, 0, 0, 0), 0, False),
     # a region's rows of 961 .. 3840 points
-    (430, 310, 9, 16, "knn", 40_000, 20, (170, 120, 70, 20), 16, False),
-    (430, 310, 9, 8, "compat", 40_000, 30, (170, 120, 90, 20), 0, False),
-    (430, 310, 10, 16, "knn", 40_000, 20, (170, 120, 70, 20), 4, True),
+    (650, 410, 9, 16, "knn", 40_000, 20, (170, 120, 70, 20), 16, False),
+    (650, 410, 9, 8, "compat", 40_000, 30, (170, 120, 90, 20), 0, False),
+    (650, 410, 10, 16, "knn", 40_000, 20, (170, 120, 70, 20), 4, True),
     # and at the image's corner, where clamping repeats them
-    (430, 310, 9, 8, "knn", 40_000, 20, (0, 0, 70, 20), 0, False),
+    (650, 410, 9, 8, "knn", 40_000, 20, (0, 0, 70, 20), 0, False),
     # rows too long for windows of up to eight columns
     (430, 310, 8, 8, "knn", 40_000, 20, (170, 120, 70, 20), 0, False),
 ]
@@ -210,6 +211,24 @@ def test_tiles(dev, case, heavy):
         assert int((out["n_samples"] > 0).sum()) > 3000
         if C.sampling_form(v.opt, len(pts), H, W, compact=False) == C.FORM_ROW_TILES:
             check_dense(v, mode)
+
+
+@pytest.mark.parametrize("case", [
+    ("thin", 515, 513, dict(radius_threshold=0.02, kernel_size=9), "compat", False, None),
+    ("thin", 515, 513, dict(t_intvl=0.0003, radius_threshold=0.02, kernel_size=9), "knn", False, None),
+    ("box", 570, 461, dict(kernel_size=16, num_point_cloud_per_sp=16), "knn", True, (torch.bfloat16, 32)),
+    ("box", 4, 65537, dict(kernel_size=15), "compat", False, (torch.float32, 4)),
+    ("hot", 513, 515, dict(kernel_size=9), "knn", False, None),
+    # windows of one and two columns, on an image of few tiles
+    ("dense", 260, 200, dict(kernel_size=1), "knn", True, None),
+    ("dense", 261, 203, dict(kernel_size=1), "compat", False, (torch.float32, 5)),
+    ("dense", 366, 359, dict(kernel_size=2), "knn", True, None),
+], ids=lambda c: f"{c[0]}-{c[1]}x{c[2]}-{c[4]}-k{c[3]['kernel_size']}")
+def test_tiles_by_window(dev, case):
+    kind, W, H, opts, _, per_point, _ = case
+    pts, _ = test_gpu_rows.scene(kind, W, H)
+    assert C.sampling_form(RenderOptions(**opts), len(pts), H, W, live=2 if per_point else None) == C.FORM_ROW_TILES
+    test_gpu_rows.test_rows_equal_lane_sets(dev, case)
 
 
 @pytest.mark.parametrize("W,H,n,form", [(200, 150, 60_000, C.FORM_ROW_WAVES), (430, 310, 120_000, C.FORM_ROW_TILES)])

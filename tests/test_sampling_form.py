@@ -45,3 +45,35 @@ def test_autotuner_varies_what_the_form_reads(monkeypatch):
     assert sorted({t["heavy"] for t in seen}) == [0, 128, 512]
     best, _ = autotune.tune("lanes", run, **autotune.knobs(C.FORM_LANE_SETS))
     assert {(t["tile_w"], t["tile_h"]) for t in seen} >= set(autotune.SHAPES)
+
+
+def test_forms_by_size():
+    """The form that measured ahead of the lane sets, or these, at each of the sizes
+    beside the rule."""
+    for n, W, H, k, want, *K in [
+        (1_400_000, 162, 93, 5, C.FORM_ROW_WAVES),
+        (50_000, 203, 152, 11, C.FORM_ROW_WAVES),
+        # few candidates, ordinary and many on small images
+        (26_667, 400, 300, 3, C.FORM_LANE_SETS),
+        (48_000, 400, 300, 5, C.FORM_ROW_TILES),
+        (263_000, 355, 357, 5, C.FORM_ROW_WAVES),
+        (2_120_000, 1448, 1449, 5, C.FORM_ROW_TILES),
+        (148_640, 963, 964, 5, C.FORM_LANE_SETS),
+        # and of rows of many neighbours
+        (135_720, 386, 292, 7, C.FORM_ROW_TILES, 32),
+        (614_280, 621, 350, 7, C.FORM_ROW_TILES, 32),
+        (614_280, 621, 350, 7, C.FORM_ROW_WAVES, 16),
+        # wide windows
+        (58_765, 400, 340, 9, C.FORM_LANE_SETS),
+        (133_926, 500, 503, 13, C.FORM_LANE_SETS),
+        (150_000, 500, 503, 9, C.FORM_LANE_SETS),
+        (682_666, 640, 480, 15, C.FORM_LANE_SETS),
+        (3_602_000, 345, 261, 9, C.FORM_ROW_WAVES),
+        (1_896_000, 640, 480, 9, C.FORM_ROW_WAVES),
+        (1_614_000, 683, 685, 9, C.FORM_LANE_SETS),
+        (1_860_000, 516, 519, 9, C.FORM_LANE_SETS, 32),
+        (398_222, 1280, 720, 9, C.FORM_ROW_TILES),
+        (20_000_000, 1920, 1080, 15, C.FORM_ROW_TILES),
+    ]:
+        K = K[0] if K else 8
+        assert form(n, W, H, kernel_size=k, num_point_cloud_per_sp=K) == want, (n, W, H, k, K)
