@@ -57,7 +57,7 @@ constexpr int kRowTileW = kWave;   // rays of a wave: consecutive columns
 constexpr int kRowTileH = 4;       // waves of a block: consecutive rows
 constexpr int kRowThreads = kRowTileW * kRowTileH;
 constexpr int kRowMaxK = 16;       // larger windows take the lane-set kernels
-constexpr int kRowCap = 960;       // points staged at once: four blocks per CU
+constexpr int kRowCap = 960;       // points staged at once: four blocks per CU, three with per-point radii
 // A row of more points than this leaves its tile's rays to waves: a piece of it
 // serves the k + 63 columns or fewer that it covers, and the others wait.
 __device__ __forceinline__ int row_longest(int k) { return k <= 8 ? kRowCap : 4 * kRowCap; }

@@ -9,7 +9,7 @@
 
 namespace epcq {
 
-constexpr int kRowWavesPerSimd = 4;    // LDS holds four blocks per CU; the registers of KMAX <= 8 do too
+constexpr int kRowWavesPerSimd = 4;    // LDS holds four blocks per CU (41.5 KB of per-point radii: three); so do the registers of KMAX <= 8
 constexpr int kRowWaveWaves = 4;       // waves of a block that takes one ray per wave
 constexpr int kDeferredBlocks = 1024;  // blocks of the deferred rays' launch
 

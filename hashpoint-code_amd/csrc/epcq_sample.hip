@@ -7,15 +7,20 @@
 //   epcq_quick_query     radius query for a ray list (:222-339)
 //   epcq_idw_features    IDW weights + weighted features (epcq/epcq.py:434-452)
 //
-// Full-image sampling runs one 256-lane block per tile of rays.  The block
-// first stages its tile's halo region -- the hash entries and bucket cones of
-// the (tw + k - 1) x (th + k - 1) neighbour pixels and, row segment by row
-// segment (contiguous in the row-major point lists), the coordinates and
-// indices of their points as float4 -- into LDS with coalesced loads; every
-// candidate walk of every ray then reads LDS.  A tile whose region holds more
-// points than the LDS capacity reads global memory instead, in the same
-// block.  Ray lists (no tile structure) read global memory.  The per-ray
-// logic is in epcq_sampler.h.
+// Sampling has three forms with the same outputs (takes_rows, takes_rows_list):
+// tiles over the rows of the point list (epcq_rows.h), one wave per ray over
+// these rows (epcq_rows_wave.h), and the lane sets.
+//
+// A lane-set image runs one 256-lane block per tile of rays.  The block first
+// stages its tile's halo region -- the hash entries and bucket cones of the
+// (tw + k - 1) x (th + k - 1) neighbour pixels and, row segment by row segment
+// (contiguous in the row-major point lists), the coordinates and indices of
+// their points as float4 -- into LDS with coalesced loads; every candidate walk
+// of every ray then reads LDS.  A tile whose region holds more points than the
+// LDS capacity, or a row that is no run of the list, reads global memory
+// instead, in the same block.  Ray lists (no tile structure) read global
+// memory, one wave or one lane per ray.  The per-ray logic of the lane sets is
+// in epcq_sampler.h.
 #include <cmath>
 #include <mutex>
 
@@ -95,9 +100,9 @@ epcq_tuning current_tuning() {
 // Pixel-ordered copy of the points, one thread per list position: (x, y,
 // z, index bits) and, with per-point radii, the radius's squared threshold.
 // Positions holding no valid index (the -1 tail) are left alone; the hash
-// entries never point there.  cand: the points' candidate bounds for the
-// row-run sampler (uniform radius r0 without prad); queue: the deferred-ray queue that the row-run
-// that sampler starts from, emptied here.
+// entries never point there.  For the row-run sampler also cand, the points'
+// candidate bounds (of the uniform radius r0 without prad), and queue, its
+// deferred rays, emptied here.
 __global__ __launch_bounds__(kBlock) void point_copy_kernel(const int* __restrict__ sorted_idx,
                                                             const float* __restrict__ xyz,
                                                             const float* __restrict__ radius, int64_t n,
@@ -438,7 +443,8 @@ void prepare_bounds(SampleOpts& o, ViewArgs& view, int64_t n, const epcq_camera*
     if (rays >= 0 && rays * o.L * kConeVisitRatio < P) return;
     if (o.rows) {
         // the row-run sampler: point copy and candidate bounds, and the queue
-        // in the cones' place (a ray list makes do with the copy alone)
+        // in the cones' place (only an image's tiles use it; a ray list whose
+        // workspace has no room for the bounds works them out on the way)
         const size_t pts_off = cone_bytes(P), rad_off = pts_off + align_up((size_t)n * 16, 256);
         const size_t cand_off = rad_off + align_up((size_t)n * 4, 256);
         if (workspace_bytes < rad_off) return;

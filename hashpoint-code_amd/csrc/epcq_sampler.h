@@ -18,9 +18,8 @@
 // occupied slots; a refill walk only when the front-to-back walk reaches a
 // slot the table does not hold; one neighbour walk per two sample points.
 // Sums are accumulated in the canonical (lane, bucket position) order, so the
-// result equals a full 128-slot histogram.  A conservative cross-product test
-// rejects candidates that are certainly outside the radius before the exact
-// projection.
+// result equals a full 128-slot histogram.  Every candidate of a bucket that its
+// cone does not clear runs the exact test.
 //
 // Candidates come from a source `Src` with
 //   int2   bucket(ub, vb)  (start, count) of pixel (ub, vb), count -1 if empty
