@@ -57,3 +57,34 @@ def test_build_takes_a_workspace_at_any_word(dev, offset):
         for size in (smallest_build(n, H, W), C.build_hashtable_workspace_size(n, H, W)):
             ws = torch.empty(offset + size, dtype=torch.uint8, device=dev)[offset:]
             same(npts.pts2plane(cs, opt, sort=sort, workspace=ws), npts.pts2plane(cs, opt, sort=sort))
+
+
+@pytest.mark.parametrize("W,H,n", [(97, 65, 60_000), (390, 350, 150_001)])
+def test_samplers_take_any_workspace(dev, monkeypatch, W, H, n):
+    """Images and ray lists, with each part of the workspace just there and just
+    missing: candidate bounds, radii, point copy, cones."""
+    npts, cs = scene(n, W, H, dev)
+    opt = RenderOptions(radius_threshold=0.012, num_point_cloud_per_sp=8, kernel_size=5)
+    idx, depth, table = npts.pts2plane(cs, opt)
+    g = torch.Generator().manual_seed(2)
+    rays = torch.randint(0, W * H, (4000,), generator=g).to(torch.int32).to(dev)
+    radius = (0.012 * torch.exp(-2.3 * torch.rand(n, generator=g))).to(dev)
+
+    def calls():
+        out = list(npts.render_image_hashtable_topk(cs, opt, idx, depth, table))
+        for kw in (dict(), dict(radius=radius, s_max=2), dict(rays=rays), dict(rays=rays, radius=radius, s_max=2)):
+            out += npts.knn_sampling(cs, opt, idx, table, mode="knn", **kw).values()
+        return out
+
+    cones = up(16 * H * W) + up(8 * H * W)
+    points, radii = cones + up(16 * n), cones + up(16 * n) + 4 * n
+    full = C._lib.epcq_sampling_workspace_size(n, H, W)
+    sizes = [full, full - 1, radii, radii - 1, points, points - 1, cones, cones - 1]
+    assert sizes == sorted(sizes, reverse=True)
+    monkeypatch.setattr(C, "_workspace", lambda *a: None)
+    want = calls()
+    assert int(want[3].sum()) > 1000
+    for size in sizes:
+        print("sampler workspace", W, H, n, size, flush=True)
+        monkeypatch.setattr(C, "_workspace", lambda *a: torch.empty(size, dtype=torch.uint8, device=dev))
+        same(calls(), want)
