@@ -517,8 +517,6 @@ __device__ __forceinline__ void row_tile_body(const SampleOpts& o, const SampleO
         const int n0 = __shfl_down(f[0], 1), n1 = __shfl_down(f[1], 1), f10 = __shfl(f[1], 0);
         if (s[0] != INT_MAX && e[0] != (lane == kWave - 1 ? f10 : n0)) flags |= kRowIrregular;
         if (s[1] != INT_MAX && e[1] != (lane == kWave - 1 ? end : n1)) flags |= kRowIrregular;
-        // nor more points than sums over the rows, which pixels may share, can count
-        if (end - __shfl(f[0], 0) > INT_MAX / kRowMaxRows) flags |= kRowIrregular;
     }
     flags = (__any(flags & kRowIrregular) ? kRowIrregular : 0) | (__any(flags & kRowBigBucket) ? kRowBigBucket : 0);
     if (lane == 0) sm.flags[wave] = flags;

@@ -379,6 +379,12 @@ constexpr int kWaveBuffer = 16;
 // five and at 0.89 from there on.
 constexpr int64_t kRowsSparse = 10, kRowsSparseCompact = 5;
 
+// The tiles add the points of a region's rows in 31 bits, and a caller's table may
+// let rows share their buckets, so that each holds up to n points.  Larger clouds
+// (113 million points at k = 16, 268 million at k = 5) take the waves, which count
+// in 63: a test in the tiles cost 20M points at 1920 x 1080 0.6 %.
+int64_t rows_most(int k) { return INT32_MAX / (kRowTileH + k - 1); }
+
 // Whether a full image takes the row-run sampler (epcq_rows.h): windows that
 // its LDS rows hold, options under which a ray can visit two slots at most
 // (with per-point radii the caller's s_max stands for that bound; a ray that
@@ -392,7 +398,7 @@ int takes_rows(SampleOpts& o, int64_t P, int64_t n, int live_bound, bool compact
     // would outlast the others
     o.row_heavy = (int)std::min<int64_t>(kRowHeavyMost, std::max<int64_t>(kRowHeavyLeast, (int64_t)o.L * n / (65536 * 128)));
     const bool wide = o.k > 8, large = o.Kc > kWaveBuffer;
-    if (P <= kWaveTiny) return kRowsWave;
+    if (P <= kWaveTiny || n > rows_most(o.k)) return kRowsWave;
     if (wide) {
         const int64_t full = (P <= 2 * kWaveImage ? kWaveFull : kWaveFullest) * (large ? 2 : 1);
         if (P <= 4 * kWaveImage && n >= full * P) return kRowsWave;

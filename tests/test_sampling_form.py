@@ -77,3 +77,12 @@ def test_forms_by_size():
     ]:
         K = K[0] if K else 8
         assert form(n, W, H, kernel_size=k, num_point_cloud_per_sp=K) == want, (n, W, H, k, K)
+
+
+def test_clouds_whose_rows_a_tile_cannot_count():
+    """The tiles add the points of k + 3 rows in 31 bits, and rows of a caller's table
+    may share their buckets."""
+    for k in (5, 8, 9, 16):
+        most = (2**31 - 1) // (k + 3)
+        assert form(most, 8000, 8000, kernel_size=k) == C.FORM_ROW_TILES
+        assert form(most + 1, 8000, 8000, kernel_size=k) == C.FORM_ROW_WAVES
