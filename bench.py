@@ -508,7 +508,7 @@ def bench_per_view(args, wl):
                    "radius": r_max, "per_point_radius": radius is not None, "K": K, "features": F,
                    "mode": args.mode, "s_max": s_max, "form": "per-view", "tuning": C.get_tuning()},
         "latency_per_view": percentiles(build_ms + sample_ms),
-        "roofline": {"bound": "hbm", "kernel": "sample_tile_kernel (knn_sampling)",
+        "roofline": {"bound": "hbm", "kernel": "sample_rows_kernel (knn_sampling)",
                      "achieved": sample_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": sample_gbs / HBM_PEAK_GBS, "traffic": None, "avg_ms": float(sample_ms.mean()),
                      "bytes_per_launch": sample_bytes},

@@ -37,13 +37,16 @@
 // rays, which come in clusters, over the whole GPU, and keeps their code out of
 // this kernel's registers.
 //
-// What bounds it: vector-instruction issue (about 10 per candidate and sweep,
-// about 60 per exact test, in which a third of the lanes take part) and, for
-// windows of many rows, the LDS reads (16 bytes per candidate and lane).
-// Measured per call with the build, against the lane-set kernels: 1M points at
-// 800 x 800, k = 5, dense layout 1.34 -> 0.74 ms; 307k points at 517 x 389,
-// k = 7, with features 1.11 -> 0.44 ms; 20M points at 1920 x 1080, k = 15,
-// with features 237 -> 24 ms.
+// What bounds it: the densest tiles, which end last, and waits.  Vector issue
+// (about 10 instructions per candidate and sweep, about 60 per exact test, in
+// which a third of the lanes take part) would take 36 % of the time for 1M points
+// at 800 x 800 (0.44 ms), 27 % for 307k at 517 x 389 (0.35 ms, 882 tiles for 1024
+// places) and 64 % for 20M at 1920 x 1080 (15.5 ms); the waves spend about half of
+// their time waiting for LDS, memory or a barrier.
+// Measured per call with the build, against the lane-set kernels and the build
+// of three arrays: 1M points at 800 x 800, k = 5, dense layout 0.89 -> 0.53 ms;
+// 307k points at 517 x 389, k = 5, with features 1.09 -> 0.42 ms; 20M points at
+// 1920 x 1080, k = 15, with features 247 -> 21.7 ms.
 #pragma once
 
 #include "epcq_sampler.h"

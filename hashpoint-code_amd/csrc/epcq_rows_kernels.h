@@ -9,7 +9,8 @@
 
 namespace epcq {
 
-constexpr int kRowWavesPerSimd = 4;    // LDS holds four blocks per CU (41.5 KB of per-point radii: three); so do the registers of KMAX <= 8
+// LDS holds four blocks per CU (three with per-point radii, 41.5 KB); the registers of KMAX <= 8 do too
+constexpr int kRowWavesPerSimd = 4;
 constexpr int kRowWaveWaves = 4;       // waves of a block that takes one ray per wave
 constexpr int kDeferredBlocks = 1024;  // blocks of the deferred rays' launch
 
