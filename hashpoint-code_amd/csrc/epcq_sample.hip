@@ -320,12 +320,6 @@ SampleOpts make_opts(const float* xyz, const epcq_options* opt, const float* rad
 
 size_t sampling_bytes(int64_t n, int64_t P);
 
-// Whether a ray list takes the one-wave-per-ray form over row runs
-// (epcq_rows_wave.h): under the same bounds, lists of at most list_wave rays.
-int takes_rows_list(const SampleOpts& o, int64_t R, int live_bound) {
-    return o.k <= kRowMaxK && live_bound <= 2 && R <= o.list_wave ? kRowsWave : kRowsNone;
-}
-
 // Which form an image takes, by its pixels P, its points n and the points d that
 // a ray's window holds on average.  The lines lie where the medians of 1,900
 // images (cameras, scenes, radii and buffers varied; call with the build, which
@@ -440,6 +434,26 @@ size_t sampling_bytes(int64_t n, int64_t P) {
 // and both ways meet near 0.24 P; on a 20M-point 1080p view with k = 15 they
 // meet near 0.2 P.  The outputs are the same either way.
 constexpr int64_t kConeVisitRatio = 4;
+
+// Whether a ray list takes the one-wave-per-ray form over row runs
+// (epcq_rows_wave.h): under the same bounds as an image, lists of at most
+// list_wave rays.  But one wave per ray over the lane sets (run_ray_wave) is ahead
+// where the buckets that it skips outweigh the cones' pass: where the windows visit
+// kListVisits buckets per pixel or more in all, and with more than 12 columns on
+// views of up to twice kWaveImage.  Rows against lane sets, medians of 2,500 lists:
+// 0.75 where the windows visit one to four buckets per pixel, 0.89 at eight to 16,
+// 0.98 at 16 to 32, 1.3 to 1.9 beyond; with more than 12 columns 1.1 to 1.2 on the
+// smaller views.  216 x 163, k = 11, 35,208 rays 0.27 / 0.14 ms; 202 x 204, k = 15,
+// 4520 rays 0.12 / 0.06; 800 x 800, k = 5, 4096 rays 0.024 / 0.057.
+constexpr int64_t kListVisits = 16;
+
+int takes_rows_list(const SampleOpts& o, int64_t R, int64_t P, int live_bound, const void* workspace,
+                    size_t workspace_bytes) {
+    if (o.k > kRowMaxK || live_bound > 2 || R > o.list_wave) return kRowsNone;
+    const bool cones = workspace && workspace_bytes >= cone_bytes(P) && R * o.L * kConeVisitRatio >= P;
+    if (cones && (R * o.L >= kListVisits * P || (o.k > 12 && P <= 2 * kWaveImage))) return kRowsNone;
+    return kRowsWave;
+}
 
 void prepare_bounds(SampleOpts& o, ViewArgs& view, int64_t n, const epcq_camera* cam, const int* sorted_idx,
                     const int* hash, void* workspace, size_t workspace_bytes, int64_t rays, hipStream_t st) {
@@ -602,8 +616,9 @@ extern "C" int32_t epcq_sampling_form(const epcq_options* opt, int64_t n, int32_
                   "the forms' numbers");
     if (!opt || height <= 0 || width <= 0 || n < 0) return EPCQ_FORM_LANE_SETS;
     SampleOpts o = make_opts(nullptr, opt, nullptr);
-    if (rays >= 0) return takes_rows_list(o, rays, live);
-    return takes_rows(o, (int64_t)height * width, n, live, compact != 0, &o, workspace_bytes);
+    const int64_t P = (int64_t)height * width;
+    if (rays >= 0) return takes_rows_list(o, rays, P, live, &o, workspace_bytes);
+    return takes_rows(o, P, n, live, compact != 0, &o, workspace_bytes);
 }
 
 extern "C" int epcq_quick_sampling(const float* xyz, int64_t n, const epcq_camera* cam, const epcq_options* opt,
@@ -649,7 +664,7 @@ extern "C" int epcq_quick_sampling_rays(const float* xyz, int64_t n, const epcq_
     if (opt->num_sample_points_per_ray == 0 || R == 0) return EPCQ_OK;
     const int bound = epcq_max_live_samples(opt, opt->radius_threshold);
     SampleOpts o = make_opts(xyz, opt, nullptr);
-    o.rows = takes_rows_list(o, R, bound);
+    o.rows = takes_rows_list(o, R, (int64_t)cam->width * cam->height, bound, workspace, workspace_bytes);
     SampleOut out{};
     out.sp_xyz = sp_xyz;
     out.pc_idx = pc_idx;
@@ -694,7 +709,8 @@ extern "C" int epcq_knn_sampling(const float* xyz, int64_t n, const epcq_camera*
     out.agg = agg;
     const int64_t nr = rays ? R : (int64_t)cam->width * cam->height;
     const int live = radius ? s_max : epcq_max_live_samples(opt, opt->radius_threshold);
-    o.rows = rays ? takes_rows_list(o, nr, live) : takes_rows(o, nr, n, live, true, workspace, workspace_bytes);
+    o.rows = rays ? takes_rows_list(o, nr, (int64_t)cam->width * cam->height, live, workspace, workspace_bytes)
+                  : takes_rows(o, nr, n, live, true, workspace, workspace_bytes);
     hipStream_t st = as_stream(stream);
     ViewArgs view = make_view(cam, sorted_idx, hash);
     prepare_bounds(o, view, n, cam, sorted_idx, hash, workspace, workspace_bytes, rays ? R : -1, st);

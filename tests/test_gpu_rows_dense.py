@@ -93,8 +93,10 @@ def test_wave_lists(dev, what, k, K, mode):
     print("wave list", what, k, K, mode, len(pts), flush=True)
     check_dense(v, mode)
     compact_vs_dense(v, mode)
-    rays = rng.integers(0, W * H, 600).astype(np.int32)
-    compact_vs_dense(v, mode, rays=rays)              # with the copy and its bounds
+    rays = rng.integers(0, W * H, 15 * W * H // k**2).astype(np.int32)
+    if k <= 12:
+        assert C.sampling_form(v.opt, len(pts), H, W, rays=len(rays)) == C.FORM_ROW_WAVES
+    compact_vs_dense(v, mode, rays=rays)              # with the copy and its bounds (k <= 12)
     compact_vs_dense(v, mode, rays=rays, cull=False)  # the bounds worked out on the way
     compact_vs_dense(v, mode, rays=rays[:3])          # a list too short for the copy
 
@@ -147,7 +149,8 @@ def test_wave_full_buckets(dev, hot, per_pixel, k, K, mode, opts):
     print("wave full buckets", hot, per_pixel, k, K, mode, flush=True)
     check_dense(v, mode)
     compact_vs_dense(v, mode)
-    rays = np.concatenate([rng.integers(0, W * H, 300), [17 * W + 22]]).astype(np.int32)
+    rays = np.concatenate([rng.integers(0, W * H, 250), [17 * W + 22]]).astype(np.int32)
+    assert C.sampling_form(v.opt, len(pts), H, W, rays=len(rays)) == C.FORM_ROW_WAVES
     feat = torch.randn(len(pts), 9, generator=torch.Generator().manual_seed(3)).to(dev)
     compact_vs_dense(v, mode, rays=rays)
     compact_vs_dense(v, mode, rays=rays, cull=False)

@@ -86,3 +86,25 @@ def test_clouds_whose_rows_a_tile_cannot_count():
         most = (2**31 - 1) // (k + 3)
         assert form(most, 8000, 8000, kernel_size=k) == C.FORM_ROW_TILES
         assert form(most + 1, 8000, 8000, kernel_size=k) == C.FORM_ROW_WAVES
+
+
+def test_lists_whose_windows_cover_the_view():
+    """Lists for which the cones' pass pays take the lane sets, where a workspace
+    holds the cones."""
+    full = lambda W, H: C._lib.epcq_sampling_workspace_size(300_000, H, W)  # noqa: E731
+    for R, W, H, k, want in [
+        (4096, 800, 800, 5, C.FORM_ROW_WAVES),
+        (25_599, 200, 200, 5, C.FORM_ROW_WAVES),
+        (25_600, 200, 200, 5, C.FORM_LANE_SETS),
+        (35_208, 216, 163, 11, C.FORM_LANE_SETS),
+        # windows of more than 12 columns: where the cones are made at all
+        (288, 512, 508, 15, C.FORM_ROW_WAVES),  # 4 * 225 * 289 buckets >= 512 * 508
+        (289, 512, 508, 15, C.FORM_LANE_SETS),
+        (2076, 551, 551, 15, C.FORM_ROW_WAVES),
+        (2076, 551, 475, 15, C.FORM_LANE_SETS),
+        (2076, 551, 475, 12, C.FORM_ROW_WAVES),
+    ]:
+        assert form(300_000, W, H, rays=R, kernel_size=k) == want, (R, W, H, k)
+        for ws in (0, W * H * 24 - 1):
+            assert ws < full(W, H)
+            assert form(300_000, W, H, rays=R, kernel_size=k, ws=ws) == C.FORM_ROW_WAVES, (R, W, H, k)
