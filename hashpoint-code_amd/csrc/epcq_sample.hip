@@ -147,8 +147,20 @@ constexpr int kQueryBucket = 1 << 24;
 // better (2513 rays of 1.4M points, 23 us, take one wave each).
 constexpr int64_t kQueryHalfWave = 16384;
 
+// Fewer lanes per ray where a ray has few outputs, so that what is left is its
+// buckets: with at most kQueryFew hits wanted, four lanes for windows of up to two
+// columns and eight for three, and from kQueryMany rays on, which fill the GPU by
+// themselves, four for up to three and eight for up to nine.  One lane per ray / 4 / 8 / 32, in ms with the
+// call's 0.02: 571k rays, k = 1, 2 hits wanted 0.025 / 0.025 / 0.039 / 0.137; 334k, k
+// = 3, 1 hit 0.024 / 0.026 / 0.031 / 0.081; 147k, k = 4, 4 hits 0.34 / 0.12 / 0.084 /
+// 0.070; but 242k, k = 5, 256 hits 0.65 / 0.30 / 0.26 / 0.22.  Over 700 calls 1.06 of
+// the best of these in the geometric mean, 1.15 without this rule.
+constexpr int kQueryFew = 32;
+constexpr int64_t kQueryMany = 131072;
+
 // hashtable_query_for_nearby_point (:222-283): hits of each neighbour bucket
-// (at most 32) appended in lane order.  G lanes take a ray: each reads the hash
+// (at most 32) appended in lane order.  G lanes take a ray, 32 or 64 of them or
+// fewer (below): each reads the hash
 // entry of one bucket, a prefix sum numbers the candidates of G buckets, and
 // the lanes take G candidates at a time, whichever bucket they are in; a ballot
 // gives each hit its place in the output, so that reads of the list and writes
@@ -738,7 +750,11 @@ extern "C" int epcq_quick_query(const float* xyz, int64_t n, const epcq_camera* 
             cam->width, cam->height, opt->kernel_size, (opt->kernel_size + 1) / 2, opt->radius_threshold, rays, R,
             opt->num_point_per_ray, out);
     };
-    if (k2 <= 32 && R >= kQueryHalfWave) launch(query_kernel<32>, 32);
+    const bool few = opt->num_point_per_ray <= kQueryFew && R >= kQueryHalfWave;
+    const bool many = R >= kQueryMany;
+    if (few && k2 <= (many ? 9 : 4)) launch(query_kernel<4>, 4);
+    else if (few && k2 <= (many ? 81 : 9)) launch(query_kernel<8>, 8);
+    else if (k2 <= 32 && R >= kQueryHalfWave) launch(query_kernel<32>, 32);
     else launch(query_kernel<64>, 64);
     return check_launch("quick_query_for_nearby_point");
 }
