@@ -1520,17 +1520,18 @@ __device__ __forceinline__ void tile_region(int W, int H, int k, int ko, int u0,
 // OWN: known to be one.
 template <bool OWN = false>
 __host__ __device__ __forceinline__ bool row_span(const int2* e, int n, int& lo, int& hi) {
-    lo = hi = 0;
-    bool found = false, ordered = true;
+    lo = INT_MAX;
+    hi = 0;
+    int behind = 0;  // negative: a bucket begins before the one to its left ends
     for (int c = 0; c < n; ++c) {
         const int2 b = e[c];
         if (b.y <= 0) continue;
-        if (!found) lo = b.x;
-        ordered = ordered && (OWN || !found || b.x >= hi);
-        found = true;
+        if (!OWN) behind |= b.x - hi;
+        lo = min(lo, b.x);
         hi = b.x + b.y;
     }
-    return ordered;
+    if (hi == 0) lo = 0;
+    return OWN || behind >= 0;
 }
 
 // Stages the halo region of the tile with top-left ray (u0, v0) into LDS:
@@ -1563,7 +1564,7 @@ __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __r
         int lo, hi;
         const bool run = row_span<OWN>(sm.hash + r * RW, RW, lo, hi);
         sm.rowlo[r] = lo;
-        sm.rowbase[r] = run ? hi - lo : INT_MAX;
+        sm.rowbase[r] = OWN ? hi - lo : run ? min(hi - lo, cap + 1) : cap + 1;
     }
     __syncthreads();
     if (tid == 0) {
@@ -1571,7 +1572,7 @@ __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __r
         for (int r = 0; r < RH; ++r) {
             const int len = sm.rowbase[r];
             sm.rowbase[r] = run;
-            run = !OWN && len > cap - run ? cap + 1 : run + len;
+            run += len;
         }
         sm.rowbase[RH] = run;
         *sm.total = run;
