@@ -1540,7 +1540,7 @@ __host__ __device__ __forceinline__ bool row_span(const int2* e, int n, int& lo,
 // region holds more than `cap` points or a row of it is no run of the list
 // (the tile then reads global memory).  OWN: the table is the library's own,
 // whose rows are runs of the list without holes, and view.pts is there: the
-// batch's pass, 1.2 % faster without the tests.
+// batch's pass, which an earlier form of the tests cost 1.2 %.
 // Block-wide; every thread of the block must call it.
 template <bool OWN>
 __device__ __forceinline__ int stage_tile(const ViewArgs& view, const float* __restrict__ xyz,
