@@ -335,9 +335,9 @@ size_t sampling_bytes(int64_t n, int64_t P);
 // Which form an image takes, by its pixels P, its points n and the points d that
 // a ray's window holds on average.  The lines lie where the medians of 1,900
 // images (cameras, scenes, radii and buffers varied; call with the build, which
-// all forms share) cross: 0.68 of the lane sets' time in the geometric mean.  A
-// twentieth of the images are more than 3 % slower than these, single ones up to
-// 1.6 times, since how the points cluster is not known here.  Tile form / wave form /
+// all forms share) cross: 0.68 of the lane sets' time in the geometric mean.  One
+// image in 25 is more than 3 % slower than these, single ones up to 1.6 times,
+// since how the points cluster is not known here.  Tile form / wave form /
 // lane sets in ms:
 // - P <= kWaveTiny: 64 rays per wave would leave SIMDs idle; waves.  260 x 147,
 //   k = 5, d = 156: 0.46 / 0.17 / 0.66; 203 x 152, k = 11, d = 202: 0.36 / 0.19 /
@@ -382,8 +382,10 @@ constexpr int kWaveBuffer = 16;
 // with 200k, 0.27 against 0.26 with 300k, 0.33 against 0.39 with 600k.  Fewer than
 // five in the compact layout: 963 x 964, k = 5, d = 4: 0.38 against 0.32, 1635 x
 // 1636, k = 3, d = 1: 0.48 against 0.36; the medians of 110 images are even below
-// five and at 0.89 from there on.
-constexpr int64_t kRowsSparse = 10, kRowsSparseCompact = 5;
+// five and at 0.89 from there on.  Fewer than 15 with six to eight columns: 1423 x
+// 1426, k = 7, d = 7: 1.06 against 0.66, 781 x 585, d = 11: 0.62 against 0.54; even in
+// the median of 32 images, 0.8 from there on.
+constexpr int64_t kRowsSparse = 10, kRowsSparseCompact = 5, kRowsSparseWide = 15;
 
 // The tiles add the points of a region's rows in 31 bits, and a caller's table may
 // let rows share their buckets, so that each holds up to n points.  Larger clouds
@@ -412,7 +414,7 @@ int takes_rows(SampleOpts& o, int64_t P, int64_t n, int live_bound, bool compact
     } else if (P <= kWaveImage && d >= (large ? kWaveMid : kWaveFew)) {
         return kRowsWave;
     }
-    if (d < (compact ? kRowsSparseCompact : kRowsSparse)) return kRowsNone;
+    if (d < (compact ? kRowsSparseCompact : kRowsSparse) || (o.k > 5 && !wide && d < kRowsSparseWide)) return kRowsNone;
     if (wide) {
         if (P <= 4 * kWaveImage) return d >= kWaveMid ? kRowsNone : kRowsTiles;
         return o.k > 12 && P <= 8 * kWaveImage && d >= kWaveMid && d < kWaveWide ? kRowsNone : kRowsTiles;

@@ -226,6 +226,7 @@ def test_tiles(dev, case, heavy):
     ("dense", 260, 200, dict(kernel_size=1), "knn", True, None),
     ("dense", 261, 203, dict(kernel_size=1), "compat", False, (torch.float32, 5)),
     ("dense", 366, 359, dict(kernel_size=2), "knn", True, None),
+    ("far", 380, 260, dict(radius_threshold=0.01, kernel_size=8), "knn", False, None),
 ], ids=lambda c: f"{c[0]}-{c[1]}x{c[2]}-{c[4]}-k{c[3]['kernel_size']}")
 def test_tiles_by_window(dev, case):
     kind, W, H, opts, _, per_point, _ = case

@@ -59,6 +59,8 @@ def test_forms_by_size():
         (263_000, 355, 357, 5, C.FORM_ROW_WAVES),
         (2_120_000, 1448, 1449, 5, C.FORM_ROW_TILES),
         (148_640, 963, 964, 5, C.FORM_LANE_SETS),
+        (100_500, 781, 585, 7, C.FORM_LANE_SETS),
+        (152_300, 781, 585, 7, C.FORM_ROW_TILES),
         # and of rows of many neighbours
         (135_720, 386, 292, 7, C.FORM_ROW_TILES, 32),
         (614_280, 621, 350, 7, C.FORM_ROW_TILES, 32),
